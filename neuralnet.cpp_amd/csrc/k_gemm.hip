@@ -1,38 +1,47 @@
-// k_gemm.hip — fp32 GEMM on the gfx950 matrix cores (v_mfma_f32_32x32x2_f32).
+// k_gemm.hip — float32 GEMM on the gfx950 bf16 matrix cores, each float32 split
+// into three bf16 parts (split_bf16.hpp: six v_mfma_f32_32x32x16_bf16 in place
+// of eight v_mfma_f32_32x32x2_f32, in 0.4 of their time, with a third of their
+// error).
 //
 // Computes C_b = alpha * op(A_b) op(B_b) for `batch` row blocks, covering
 // ComputeEngine::matmul (compute_engine.hpp:182-184) and ::batched_matmul
 // (:195-199; cpu_engine.hpp:335-419 applies alpha after the product, so does
 // the epilogue here). All four transpose combinations are handled at the
-// global->LDS staging step: both operands are kept k-major in LDS
-// (As[k][m], Bs[k][n]) so every MFMA fragment read is 32 consecutive floats.
+// global->LDS staging step: a thread holds 8 k of one row of A or column of B,
+// splits them and writes each part's 16 bytes, so the LDS holds both operands
+// k-contiguous and an MFMA operand is one ds_read_b128.
 //
 // Tiling: a workgroup of WM x WN waves owns a (32*FM*WM) x (32*FN*WN) tile of
-// C; each wave owns FM x FN MFMA 32x32 blocks (64 x 64 or 32 x 64).
-// K advances 16 at a time through two LDS buffers: the next stage's global
-// loads are issued into registers before the current stage's MFMAs and
-// written to the other buffer afterwards (one barrier per stage). Tile ids are
-// remapped so that each XCD (own L2) works on a contiguous, row-grouped slab.
-// Small output grids with long K (weight gradients) split K across
-// workgroups; the partial tiles are summed in order (deterministic).
+// C; each wave owns FM x FN MFMA 32x32 blocks, 64 x 64 where the size allows:
+// per k of 16 that is 12 LDS reads for 24 MFMAs (64 of the CU's 128 bytes a
+// cycle) and 128 accumulator registers, two waves a SIMD. What bounds it: the
+// matrix cores (six products of the work), and beside them the split, 4.5
+// vector instructions an element staged (1/128 + 1/256 elements a product in
+// the 256 x 128 tile). K advances 32 at a time. 256 x 128 tiles (8 waves, one
+// workgroup a CU) have two LDS buffers and convert stage k + 1 in the shadow
+// of stage k's MFMAs, with stage k + 2's loads in flight; the 4-wave tiles
+// have one buffer, so that two or three workgroups share a CU and cover each
+// other's conversions. Measured on MI355X, float32 MFMA before -> now:
+// 6144 x 8192 x 768 126 -> 186 TFLOP/s, 4096^3 126 -> 204. The same loop
+// without the conversions runs 210 and 237; the bf16 cores alone would give
+// 348. Tile ids are remapped so that each XCD (own L2) works on a contiguous,
+// row-grouped slab. Small output grids with long K (weight gradients) split K
+// across workgroups; the partial tiles are summed in order (deterministic).
 //
-// MFMA 32x32x2 f32 operand layout (per lane l, k-step of 2):
-//   A: A[i = l%32][k = l/32],  B: B[k = l/32][j = l%32],
+// MFMA 32x32x16 bf16 operand layout (per lane l, k-step of 16):
+//   A: A[i = l%32][k = 8*(l/32) + 0..7],  B: B[k = 8*(l/32) + 0..7][j = l%32],
 //   D: 16 values, value r at row 8*(r/4) + 4*(l/32) + r%4, column l%32.
 #include <cmath>
 #include <mutex>
 
 #include "common.hpp"
 #include "nnhip_kernels.h"
+#include "split_bf16.hpp"
 
 namespace nnhip
 {
 namespace
 {
-
-typedef float floatx16 __attribute__((ext_vector_type(16)));
-
-constexpr int PAD = 4;
 
 // Tile id for workgroup `bid` of `nt` tiles (tiles_m x tiles_n). Workgroups are
 // dispatched round-robin over the 8 XCDs, each with its own L2: the remap
@@ -50,8 +59,6 @@ __device__ __forceinline__ void tile_coords(int bid, int nt, int tiles_m, int ti
     tm = first_m + r % gsize;
     tn = r / gsize;
 }
-
-typedef float f4 __attribute__((ext_vector_type(4)));
 
 // Up to four products of one shape (the attention's q, k, v projections of
 // one input; the weight gradients of its four Linears): workgroup batch z takes
@@ -91,40 +98,166 @@ struct RowSums
     int acc;
 };
 
+// One workgroup's view of an operand: ROWS of its lines (rows of A, columns of
+// B) by BK of k a stage, held by the threads as units of one line x 8 k. KC:
+// stored with k contiguous (an untransposed A, a transposed B): a unit is two
+// 16-byte loads and four neighbouring threads read one line's 32 k. Otherwise
+// the lines are contiguous: a unit is eight 4-byte loads, each of them one
+// whole run of a wave's 64 lines, and the unit comes out with its 8 k in one
+// thread all the same, as the LDS holds them. Loads need 4-byte alignment
+// only. Lines past the last are read from the last one (their outputs are not
+// stored); k from k_hi on is zero.
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+constexpr int BK = 32;
+
+template <bool KC, int ROWS, int NT>
+struct Operand
+{
+    static constexpr int U = ROWS * (BK / 8) / NT;
+    static_assert(U * NT == ROWS * (BK / 8), "tile not divisible by the workgroup");
+    static_assert(!KC || NT % 4 == 0, "four threads a line");
+    static_assert(KC || (ROWS % 64 == 0 && NT % ROWS == 0), "a wave's lanes share one k");
+    floatx8 r[U];
+    const float* p[KC ? U : 1];   // KC: each unit's line at the stage's k
+    const float* base;            // else: the operand at line 0, k 0
+    long ld, off;                 // else: off: added to every line (by sequence: the tile's sequence)
+    int line;                     // else: the thread's line (clamped)
+    int k_in, T;                  // KC by sequence: k within the sequence, its length (0: plain)
+    long step;                    // its extra offset per sequence
+
+    static __device__ __forceinline__ int unit_line(int u) { return KC ? (threadIdx.x + NT * u) / 4 : threadIdx.x % ROWS; }
+    static __device__ __forceinline__ int unit_k(int u)
+    {
+        if constexpr (KC) return 8 * (threadIdx.x % 4);
+        else return 8 * __builtin_amdgcn_readfirstlane((threadIdx.x + NT * u) / ROWS);
+    }
+    __device__ __forceinline__ void init(const float* q, long ld_, int line0, int lines, int k_lo, int T_, long step_,
+                                         long off_)
+    {
+        base = q;
+        ld = ld_;
+        off = off_;
+        T = T_;
+        step = step_;
+        if constexpr (KC)
+        {
+            int k = k_lo + unit_k(0);
+            long at = k;
+            if (T)
+            {
+                at += (long)(k / T) * step;
+                k_in = k % T;
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) p[u] = q + (long)min(line0 + unit_line(u), lines - 1) * ld + at;
+        }
+        else
+            line = min(line0 + unit_line(0), lines - 1);
+    }
+    // The stage at k0 (which KC's pointers stand at, and move past); `tail`: it may reach past k_hi.
+    template <class Seg>
+    __device__ __forceinline__ void load(int k0, int k_hi, bool tail, const Seg& seg)
+    {
+        if constexpr (KC)
+        {
+            const int left = k_hi - (k0 + unit_k(0));
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+            {
+                if (!tail || left >= 8)
+                {
+                    const f4u x = *reinterpret_cast<const f4u*>(p[u]), y = *reinterpret_cast<const f4u*>(p[u] + 4);
+                    r[u] = floatx8{x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]};
+                }
+                else
+                {
+#pragma unroll
+                    for (int q = 0; q < 8; ++q) r[u][q] = q < left ? p[u][q] : 0.0f;
+                }
+                p[u] += BK;
+            }
+            if (T)
+            {
+                k_in += BK;
+                while (k_in >= T)
+                {
+                    k_in -= T;
+#pragma unroll
+                    for (int u = 0; u < U; ++u) p[u] += step;
+                }
+            }
+        }
+        else
+        {
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+            {
+                const int k = k0 + unit_k(u), left = k_hi - k;
+                if (!tail || left >= 8)
+                {
+                    const float* q0 = seg(base, k) + off + (long)seg.within(k) * ld;
+#pragma unroll
+                    for (int q = 0; q < 8; ++q) r[u][q] = (q0 + (long)q * ld)[line];
+                }
+                else
+                {
+                    r[u] = floatx8{};
+                    if (left > 0)
+                    {
+                        const float* q0 = seg(base, k) + off + (long)seg.within(k) * ld;
+#pragma unroll
+                        for (int q = 0; q < 8; ++q)
+                            if (q < left) r[u][q] = (q0 + (long)q * ld)[line];
+                    }
+                }
+            }
+        }
+    }
+};
+
+// LDS place of 8 k (slot s of 4) of a line: lines of 64 bytes, the slots
+// swapped so that 16 neighbouring lines' same slot covers the 64 banks once.
+__device__ __forceinline__ int lds_slot(int line, int s) { return line * 4 + (s ^ ((line >> 2) & 3)); }
+
+// Whole products and sums of KSEG segments (k runs through operand k / klen).
+struct SegNone
+{
+    __device__ __forceinline__ const float* operator()(const float* whole, int) const { return whole; }
+    __device__ __forceinline__ int within(int k) const { return k; }
+};
+struct SegList
+{
+    const float* const* ops;
+    int klen;
+    // (at most kGroupMax segments: comparisons in place of a division)
+    __device__ __forceinline__ int index(int k) const { return (k >= klen) + (k >= 2 * klen) + (k >= 3 * klen); }
+    __device__ __forceinline__ const float* operator()(const float*, int k) const { return ops[index(k)]; }
+    __device__ __forceinline__ int within(int k) const { return k - index(k) * klen; }
+};
+
 // WM x WN waves; each wave owns (32*FM) x (32*FN) of C as FM x FN MFMA 32x32 blocks.
+// NBUF: LDS buffers of a stage (two: conversion of the next one beside the MFMAs).
 // STATS: besides C, each workgroup writes the column softmax statistics of its
 // BM rows of C (as stored, bias included): part[tile_m * N + n] = max over the
 // rows, part[(tiles_m + tile_m) * N + n] = sum of exp(c - max) over them. The
 // sparse cross-entropy that follows the product (the GPT's lm_head logits)
 // merges these instead of reading C once more for them. Needs splits == 1.
-template <int WM, int WN, int FM, int FN, int BK, bool TA, bool TB, bool GUARD, bool STATS = false, bool GRP = false,
+template <int WM, int WN, int FM, int FN, int NBUF, bool TA, bool TB, bool STATS = false, bool GRP = false,
           bool KSEG = false, bool RSUM = false, bool SEG = false>
-__global__ __launch_bounds__(64 * WM * WN) void k_gemm(const float* __restrict__ A, const float* __restrict__ B,
-                                                       float* __restrict__ C, int M, int N, int K, long lda, long ldb,
-                                                       long strideA, long strideB, long strideC, float alpha,
-                                                       int tiles_m, int tiles_n, int k_split, float* __restrict__ part,
-                                                       const float* __restrict__ bias, int accum, GemmGroup grp,
-                                                       RowSums rs = {})
+__global__ __launch_bounds__(64 * WM * WN, FM * FN == 4 ? 2 : FM * FN == 2 ? 3 : 4) void k_gemm(
+    const float* __restrict__ A, const float* __restrict__ B, float* __restrict__ C, int M, int N, int K, long lda,
+    long ldb, long strideA, long strideB, long strideC, float alpha, int tiles_m, int tiles_n, int k_split,
+    float* __restrict__ part, const float* __restrict__ bias, int accum, GemmGroup grp, RowSums rs)
 {
     static_assert(!RSUM || (GRP && !TA), "row sums of an untransposed A in grouped launches");
-    static_assert(!SEG || (!GUARD && !STATS), "operands by sequence in whole tiles only");
+    static_assert(!SEG || !STATS, "no column statistics of operands by sequence");
     constexpr int NT = 64 * WM * WN;
     constexpr int BM = 32 * FM * WM, BN = 32 * FN * WN;
-    constexpr int LA = BM * BK / 4 / NT;   // float4 per thread per stage for A
-    constexpr int LB = BN * BK / 4 / NT;
-    static_assert(LA * 4 * NT == BM * BK && LB * 4 * NT == BN * BK, "tile not divisible by the workgroup");
-    // An A contiguous in k (untransposed) is staged as it lies, [m][k] (one
-    // 16-byte LDS write per float4); a transposed A and B are staged k-major.
-    // Within a stage the MFMA steps take k in the order k = 8 * (lane / 32) +
-    // step, so a lane's eight k of one row of A are adjacent (two 16-byte LDS
-    // reads); B uses the same order. Measured on the GPT-step products (d 768,
-    // 8192 tokens): NN 101 -> 105 and 113 -> 117 TFLOP/s; staging a transposed
-    // B as [n][k] as well was 3-5 % slower on the weight-gradient (NT) products.
-    constexpr bool AK = !TA;
-    constexpr int KROW = BK + 4;   // [m][k] row stride: 8 rows cover all 32 banks
-    constexpr int A_R = AK ? BM : BK, A_C = AK ? KROW : BM + PAD;
-    __shared__ __attribute__((aligned(16))) float As[2][A_R][A_C];
-    __shared__ __attribute__((aligned(16))) float Bs[2][BK][BN + PAD];
+    constexpr int SLOTS = BK / 8;
+    typedef Operand<!TA, BM, NT> OpA;
+    typedef Operand<TB, BN, NT> OpB;
+    __shared__ __attribute__((aligned(16))) bf16x8 As[NBUF][3][BM * SLOTS];
+    __shared__ __attribute__((aligned(16))) bf16x8 Bs[NBUF][3][BN * SLOTS];
 
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = tid >> 6;
@@ -155,7 +288,7 @@ __global__ __launch_bounds__(64 * WM * WN) void k_gemm(const float* __restrict__
     if (!STATS && gridDim.y > 1) C = part + ((long)blockIdx.y * gridDim.z + bz) * strideC;
     // SEG: the member's sequence layouts (extra offset per sequence: step - T)
     int sa_t = 0, sb_t = 0;
-    long sa_d = 0, sb_d = 0, b_off = 0;
+    long sa_d = 0, sb_d = 0;
     if constexpr (SEG)
     {
         const int gi = GRP ? static_cast<int>(bz / grp.nb) : 0;
@@ -165,187 +298,149 @@ __global__ __launch_bounds__(64 * WM * WN) void k_gemm(const float* __restrict__
         sb_d = grp.bS[gi] - sb_t;
         if (sa_t) lda = sa_t;   // rows of a sequence-stored operand are T apart
         if (sb_t) ldb = sb_t;
-        if (!TB && sb_t) b_off = (long)(n0 / sb_t) * sb_d;
     }
+    // An untransposed B by sequence: its columns of this tile lie in one sequence.
+    const long b_off = SEG && !TB && sb_t ? (long)(n0 / sb_t) * sb_d : 0;
+    auto segs = [&](const float* const* ops) {
+        if constexpr (KSEG) return SegList{ops, grp.klen};
+        else return SegNone{};
+    };
+    const auto seg_a = segs(grp.A);
+    const auto seg_b = segs(grp.B);
 
-    f4 ra[LA], rb[LB];   // native vectors: HIP's float4 struct kept these arrays in scratch
-
-    // KSEG: the operands of the segment holding stage k0 (a stage never
-    // straddles two: klen % BK == 0), addressed with k within the segment.
-    auto seg_of = [&](int k0, const float* const* ops, const float* whole, int& kb) {
-        if constexpr (KSEG)
-        {
-            const int sg = k0 / grp.klen;
-            kb = k0 - sg * grp.klen;
-            return ops[sg];
-        }
-        kb = k0;
-        return whole;
+    OpA oa;
+    OpB ob;
+    oa.init(A, lda, m0, M, k_lo, SEG && !TA ? sa_t : 0, sa_d, 0);
+    ob.init(B, ldb, n0, N, k_lo, SEG && TB ? sb_t : 0, sb_d, b_off);
+    auto load = [&](int kt, bool tail) {
+        oa.load(k_lo + kt * BK, k_hi, tail, seg_a);
+        ob.load(k_lo + kt * BK, k_hi, tail, seg_b);
     };
-    // A_eff(m, k) = TA ? A[k*lda + m] : A[m*lda + k]
-    auto load_a = [&](int k0) {
-        int kb;
-        const float* Ap = seg_of(k0, grp.A, A, kb);
-        if constexpr (SEG && !TA)
-            if (sa_t) Ap += (long)(kb / sa_t) * sa_d;
-#pragma unroll
-        for (int s = 0; s < LA; ++s)
-        {
-            const int idx = tid + NT * s;
-            int m, k;
-            if constexpr (TA) { k = idx / (BM / 4); m = (idx % (BM / 4)) * 4; }
-            else { m = idx / (BK / 4); k = (idx % (BK / 4)) * 4; }
-            const int gm = m0 + m, gk = kb + k, dk = k0 - kb;   // gk + dk: k over the whole sum
-            if constexpr (!GUARD)
-            {
-                ra[s] = TA ? *reinterpret_cast<const f4*>(Ap + (long)gk * lda + gm)
-                           : *reinterpret_cast<const f4*>(Ap + (long)gm * lda + gk);
-            }
-            else
-            {
-                float v[4];
-#pragma unroll
-                for (int q = 0; q < 4; ++q)
-                {
-                    const int mm = TA ? gm + q : gm, kk = TA ? gk : gk + q;
-                    v[q] = (mm < M && kk + dk < k_hi) ? (TA ? Ap[(long)kk * lda + mm] : Ap[(long)mm * lda + kk])
-                                                       : 0.0f;
-                }
-                ra[s] = f4{v[0], v[1], v[2], v[3]};
-            }
-        }
-    };
-    // B_eff(k, n) = TB ? B[n*ldb + k] : B[k*ldb + n]
-    auto load_b = [&](int k0) {
-        int kb;
-        const float* Bp = seg_of(k0, grp.B, B, kb);
-        if constexpr (SEG)
-        {
-            if (!TB) Bp += b_off;
-            else if (sb_t) Bp += (long)(kb / sb_t) * sb_d;
-        }
-#pragma unroll
-        for (int s = 0; s < LB; ++s)
-        {
-            const int idx = tid + NT * s;
-            int n, k;
-            if constexpr (!TB) { k = idx / (BN / 4); n = (idx % (BN / 4)) * 4; }
-            else { n = idx / (BK / 4); k = (idx % (BK / 4)) * 4; }
-            const int gn = n0 + n, gk = kb + k, dk = k0 - kb;
-            if constexpr (!GUARD)
-            {
-                rb[s] = !TB ? *reinterpret_cast<const f4*>(Bp + (long)gk * ldb + gn)
-                            : *reinterpret_cast<const f4*>(Bp + (long)gn * ldb + gk);
-            }
-            else
-            {
-                float v[4];
-#pragma unroll
-                for (int q = 0; q < 4; ++q)
-                {
-                    const int nn = !TB ? gn + q : gn, kk = !TB ? gk : gk + q;
-                    v[q] = (nn < N && kk + dk < k_hi) ? (!TB ? Bp[(long)kk * ldb + nn] : Bp[(long)nn * ldb + kk])
-                                                       : 0.0f;
-                }
-                rb[s] = f4{v[0], v[1], v[2], v[3]};
-            }
-        }
-    };
-    float racc[RSUM ? LA : 1] = {};
+    const SplitUnits su;
+    float racc[RSUM ? OpA::U : 1] = {};
     const bool rsum_here = RSUM && tni == 0;
-    auto store_a = [&](int buf) {
+    auto store = [&](int buf) {
         if constexpr (RSUM)
             if (rsum_here)
             {
 #pragma unroll
-                for (int s = 0; s < LA; ++s) racc[s] += (ra[s].x + ra[s].y) + (ra[s].z + ra[s].w);
+                for (int u = 0; u < OpA::U; ++u)
+                    racc[u] += ((oa.r[u][0] + oa.r[u][1]) + (oa.r[u][2] + oa.r[u][3])) +
+                               ((oa.r[u][4] + oa.r[u][5]) + (oa.r[u][6] + oa.r[u][7]));
             }
 #pragma unroll
-        for (int s = 0; s < LA; ++s)
+        for (int u = 0; u < OpA::U; ++u)
         {
-            const int idx = tid + NT * s;
-            if constexpr (TA)
-            {
-                const int k = idx / (BM / 4), m = (idx % (BM / 4)) * 4;
-                *reinterpret_cast<f4*>(&As[buf][k][m]) = ra[s];
-            }
-            else
-            {
-                const int m = idx / (BK / 4), k = (idx % (BK / 4)) * 4;
-                *reinterpret_cast<f4*>(&As[buf][m][k]) = ra[s];
-            }
+            const int o = lds_slot(OpA::unit_line(u), OpA::unit_k(u) / 8);
+            split3(su, oa.r[u], As[buf][0][o], As[buf][1][o], As[buf][2][o]);
         }
-    };
-    auto store_b = [&](int buf) {
 #pragma unroll
-        for (int s = 0; s < LB; ++s)
+        for (int u = 0; u < OpB::U; ++u)
         {
-            const int idx = tid + NT * s;
-            if constexpr (!TB)
-            {
-                const int k = idx / (BN / 4), n = (idx % (BN / 4)) * 4;
-                *reinterpret_cast<f4*>(&Bs[buf][k][n]) = rb[s];
-            }
-            else
-            {
-                const int n = idx / (BK / 4), k = (idx % (BK / 4)) * 4;
-                Bs[buf][k + 0][n] = rb[s].x;
-                Bs[buf][k + 1][n] = rb[s].y;
-                Bs[buf][k + 2][n] = rb[s].z;
-                Bs[buf][k + 3][n] = rb[s].w;
-            }
+            const int o = lds_slot(OpB::unit_line(u), OpB::unit_k(u) / 8);
+            split3(su, ob.r[u], Bs[buf][0][o], Bs[buf][1][o], Bs[buf][2][o]);
         }
     };
 
-    floatx16 acc[FM][FN];
+    floatx16 acc[FM][FN] = {}, small[FM][FN] = {};
+    const int al = wm * 32 * FM + (lane & 31), bl = wn * 32 * FN + (lane & 31), kl = lane >> 5;
+    auto products = [&](int buf) {
+#pragma unroll
+        for (int kk = 0; kk < BK / 16; ++kk)
+        {
+            bf16x8 a[FM][3], b[FN][3];
+#pragma unroll
+            for (int i = 0; i < FM; ++i)
+#pragma unroll
+                for (int p = 0; p < 3; ++p) a[i][p] = As[buf][p][lds_slot(al + 32 * i, 2 * kk + kl)];
+#pragma unroll
+            for (int j = 0; j < FN; ++j)
+#pragma unroll
+                for (int p = 0; p < 3; ++p) b[j][p] = Bs[buf][p][lds_slot(bl + 32 * j, 2 * kk + kl)];
+            mfma_split(a, b, acc, small);
+        }
+    };
+
+    const int nk = (k_hi - k_lo + BK - 1) / BK;
+    const int full = (k_hi - k_lo) / BK;   // stages that hold BK of k each
+    if (nk > 0) load(0, full == 0);
+    if constexpr (NBUF == 2)
+    {
+        if (nk > 0)
+        {
+            store(0);
+            if (nk > 1) load(1, full < 2);
+            __syncthreads();
+            int kt = 0;
+            for (; kt + 2 < full; ++kt)
+            {
+                // one block of straight code: the conversion and the LDS writes
+                // of stage kt + 1 issue in the shadow of stage kt's MFMAs
+                store((kt & 1) ^ 1);
+                load(kt + 2, false);
+                products(kt & 1);
+                __syncthreads();
+            }
+            for (; kt < nk; ++kt)
+            {
+                if (kt + 1 < nk) store((kt & 1) ^ 1);
+                if (kt + 2 < nk) load(kt + 2, kt + 2 >= full);
+                products(kt & 1);
+                __syncthreads();
+            }
+        }
+    }
+    else
+        for (int kt = 0; kt < nk; ++kt)
+        {
+            store(0);
+            __syncthreads();
+            if (kt + 1 < nk) load(kt + 1, kt + 1 >= full);
+            products(0);
+            __syncthreads();
+        }
+
+    // The wave's values, or, where one is not finite, the same sums on the
+    // float32 matrix cores straight from memory (overflow of the scaled parts,
+    // infinities and NaN: as those cores give them).
+    float check = 0.0f;
 #pragma unroll
     for (int i = 0; i < FM; ++i)
 #pragma unroll
         for (int j = 0; j < FN; ++j)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
-
-    const int kt_n = (k_hi - k_lo + BK - 1) / BK;
-    if (kt_n > 0)
+            for (int r = 0; r < 16; ++r)
+            {
+                acc[i][j][r] = kSplitUnscale * (acc[i][j][r] + small[i][j][r]);
+                check = __builtin_fmaf(acc[i][j][r], 0.0f, check);
+            }
+    if (__any(check != 0.0f))
     {
-        load_a(k_lo);
-        load_b(k_lo);
-        store_a(0);
-        store_b(0);
-        __syncthreads();
-    }
-    const int am = wm * 32 * FM + (lane & 31), bn = wn * 32 * FN + (lane & 31), kl = lane >> 5;
-    for (int kt = 0; kt < kt_n; ++kt)
-    {
-        const int buf = kt & 1;
-        const bool more = kt + 1 < kt_n;
-        if (more)
-        {
-            load_a(k_lo + (kt + 1) * BK);
-            load_b(k_lo + (kt + 1) * BK);
-        }
-        static_assert(BK == 16, "k order assumes 8 MFMA steps per stage");
+        const int am = m0 + al, bn = n0 + bl;
 #pragma unroll
-        for (int kk = 0; kk < 8; ++kk)
-        {
-            const int k = 8 * kl + kk;
-            float a[FM], b[FN];
+        for (int i = 0; i < FM; ++i)
 #pragma unroll
-            for (int i = 0; i < FM; ++i) a[i] = AK ? As[buf][am + 32 * i][k] : As[buf][k][am + 32 * i];
-#pragma unroll
-            for (int j = 0; j < FN; ++j) b[j] = Bs[buf][k][bn + 32 * j];
-#pragma unroll
-            for (int i = 0; i < FM; ++i)
-#pragma unroll
-                for (int j = 0; j < FN; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], b[j], acc[i][j], 0, 0, 0);
-        }
-        if (more)
-        {
-            store_a(buf ^ 1);
-            store_b(buf ^ 1);
-        }
-        __syncthreads();
+            for (int j = 0; j < FN; ++j)
+            {
+                floatx16 c = {};
+                const long gm = min(am + 32 * i, M - 1), gn = min(bn + 32 * j, N - 1);
+                for (int k0 = k_lo; k0 < k_hi; k0 += 2)
+                {
+                    const int k = k0 + kl;
+                    float a = 0.0f, b = 0.0f;
+                    if (k < k_hi)
+                    {
+                        const float* ap = seg_a(A, k);
+                        const float* bp = seg_b(B, k) + b_off;
+                        const long ka = seg_a.within(k) + (SEG && !TA && sa_t ? (long)(k / sa_t) * sa_d : 0);
+                        const long kb = seg_b.within(k) + (SEG && TB && sb_t ? (long)(k / sb_t) * sb_d : 0);
+                        a = TA ? ap[ka * lda + gm] : ap[gm * lda + ka];
+                        b = TB ? bp[gn * ldb + kb] : bp[kb * ldb + gn];
+                    }
+                    c = __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
+                }
+                acc[i][j] = c;
+            }
     }
 
     // Epilogue: C = alpha * acc, then + bias[row] and / or + C (each rounded
@@ -363,7 +458,7 @@ __global__ __launch_bounds__(64 * WM * WN) void k_gemm(const float* __restrict__
             for (int r = 0; r < 16; ++r)
             {
                 const int gm = m0 + wm * 32 * FM + i * 32 + 8 * (r / 4) + row_l + (r % 4);
-                const float bv = (bias && (!GUARD || gm < M)) ? bias[gm] : 0.0f;
+                const float bv = (bias && gm < M) ? bias[gm] : 0.0f;
 #pragma unroll
                 for (int j = 0; j < FN; ++j)
                 {
@@ -373,7 +468,7 @@ __global__ __launch_bounds__(64 * WM * WN) void k_gemm(const float* __restrict__
                     acc[i][j][r] = v;
                 }
             }
-        float* sm = &Bs[0][0][0];    // [WM][BN] maxima, then [WM][BN] sums (the stages are done)
+        float* sm = reinterpret_cast<float*>(&Bs[0][0][0]);    // [WM][BN] maxima, then [WM][BN] sums (the stages are done)
         float* ss = sm + WM * BN;
 #pragma unroll
         for (int j = 0; j < FN; ++j)
@@ -385,7 +480,7 @@ __global__ __launch_bounds__(64 * WM * WN) void k_gemm(const float* __restrict__
                 for (int r = 0; r < 16; ++r)
                 {
                     const int gm = m0 + wm * 32 * FM + i * 32 + 8 * (r / 4) + row_l + (r % 4);
-                    if (!GUARD || gm < M) mx = fmaxf(mx, acc[i][j][r]);
+                    if (gm < M) mx = fmaxf(mx, acc[i][j][r]);
                 }
             mx = fmaxf(mx, __shfl_xor(mx, 32, 64));   // lanes l and l ^ 32 hold one column's other rows
             float sum = 0.0f;
@@ -396,7 +491,7 @@ __global__ __launch_bounds__(64 * WM * WN) void k_gemm(const float* __restrict__
                     for (int r = 0; r < 16; ++r)
                     {
                         const int gm = m0 + wm * 32 * FM + i * 32 + 8 * (r / 4) + row_l + (r % 4);
-                        if (!GUARD || gm < M) sum += __expf(acc[i][j][r] - mx);
+                        if (gm < M) sum += __expf(acc[i][j][r] - mx);
                     }
             sum += __shfl_xor(sum, 32, 64);
             if (lane < 32)
@@ -409,7 +504,7 @@ __global__ __launch_bounds__(64 * WM * WN) void k_gemm(const float* __restrict__
         for (int c = tid; c < BN; c += NT)
         {
             const int gn = n0 + c;
-            if (GUARD && gn >= N) continue;
+            if (gn >= N) continue;
             float m = sm[c], t = ss[c];
             for (int w = 1; w < WM; ++w)   // merge the waves' row bands in row order
             {
@@ -433,10 +528,10 @@ __global__ __launch_bounds__(64 * WM * WN) void k_gemm(const float* __restrict__
     const float* bsh = nullptr;
     if (!plain && bias)
     {
-        float* bl = &As[0][0][0];
-        for (int m = tid; m < BM; m += NT) bl[m] = (!GUARD || m0 + m < M) ? bias[m0 + m] : 0.0f;
+        float* bv = reinterpret_cast<float*>(&As[0][0][0]);
+        for (int m = tid; m < BM; m += NT) bv[m] = m0 + m < M ? bias[m0 + m] : 0.0f;
         __syncthreads();
-        bsh = bl;
+        bsh = bv;
     }
 #pragma unroll
     for (int i = 0; i < FM; ++i)
@@ -448,7 +543,7 @@ __global__ __launch_bounds__(64 * WM * WN) void k_gemm(const float* __restrict__
             for (int r = 0; r < 16; ++r)
             {
                 const int ml = wm * 32 * FM + i * 32 + 8 * (r / 4) + row_l + (r % 4), gm = m0 + ml;
-                if (GUARD && !(gm < M && gn < N)) continue;
+                if (!(gm < M && gn < N)) continue;
                 float* c = C + (long)gm * N + gn;
                 if (plain)
                 {
@@ -467,16 +562,16 @@ __global__ __launch_bounds__(64 * WM * WN) void k_gemm(const float* __restrict__
     if constexpr (RSUM)
         if (rsum_here)
         {
-            // the BK / 4 threads that stage one row's float4s of a stage are adjacent lanes
-            static_assert(BK / 4 == 4 && NT % 64 == 0, "row-sum lanes");
+            // the four threads that hold one row's units of a stage are adjacent lanes
+            static_assert(BK / 8 == 4 && NT % 64 == 0, "row-sum lanes");
             const long gi = bz / grp.nb;
 #pragma unroll
-            for (int s = 0; s < LA; ++s)
+            for (int u = 0; u < OpA::U; ++u)
             {
-                float v = racc[s];
+                float v = racc[u];
                 v += __shfl_xor(v, 1, 64);
                 v += __shfl_xor(v, 2, 64);
-                const int gm = m0 + (tid + NT * s) / (BK / 4);
+                const int gm = m0 + OpA::unit_line(u);
                 if ((tid & 3) != 0 || gm >= M) continue;
                 if (gridDim.y > 1)
                     rs.part[((long)blockIdx.y * gridDim.z + bz) * M + gm] = v;
@@ -768,117 +863,63 @@ struct Epi
     bool by_seq = false;                // the group passed (grp, seg or sq) holds sequence layouts
 };
 
-template <int WM, int WN, int FM, int FN, int BK, bool TA, bool TB>
+template <int WM, int WN, int FM, int FN, int NBUF, bool TA, bool TB>
 void launch_cfg(const float* A, const float* B, float* C, int M, int N, int K, long lda, long ldb, long sA, long sB,
-                long sC, float alpha, int batch, bool vec_ok, int splits, int k_split, float* part, hipStream_t s,
-                Epi e)
+                long sC, float alpha, int batch, int splits, int k_split, float* part, hipStream_t s, Epi e)
 {
     constexpr int BM = 32 * FM * WM, BN = 32 * FN * WN;
     const int tm = (M + BM - 1) / BM, tn = (N + BN - 1) / BN;
-    const bool guard = !vec_ok || (M % BM) || (N % BN) || (K % BK) || (k_split % BK);
     const dim3 grid(static_cast<unsigned>(tm * tn), static_cast<unsigned>(splits), static_cast<unsigned>(batch));
     const dim3 block(64 * WM * WN);
-    if (e.by_seq)
-    {
-        if constexpr (TA && !TB)
-            if (e.seg && !guard)
-                hipLaunchKernelGGL((k_gemm<WM, WN, FM, FN, BK, TA, TB, false, false, false, true, false, true>), grid,
-                                   block, 0, s, A, B, C, M, N, K, lda, ldb, sA, sB, sC, alpha, tm, tn, k_split, part,
-                                   e.bias, e.accum, *e.seg);
-        if constexpr (!TA && TB)
-            if (e.grp && !guard)
-            {
-                if (e.rs)
-                    hipLaunchKernelGGL((k_gemm<WM, WN, FM, FN, BK, TA, TB, false, false, true, false, true, true>), grid,
-                                       block, 0, s, A, B, C, M, N, K, lda, ldb, sA, sB, sC, alpha, tm, tn, k_split,
-                                       part, e.bias, e.accum, *e.grp, *e.rs);
-                else
-                    hipLaunchKernelGGL((k_gemm<WM, WN, FM, FN, BK, TA, TB, false, false, true, false, false, true>),
-                                       grid, block, 0, s, A, B, C, M, N, K, lda, ldb, sA, sB, sC, alpha, tm, tn, k_split,
-                                       part, e.bias, e.accum, *e.grp, RowSums{});
-            }
-        if constexpr (!TA && !TB)
-            if (e.sq && !guard)
-                hipLaunchKernelGGL((k_gemm<WM, WN, FM, FN, BK, TA, TB, false, false, false, false, false, true>), grid,
-                                   block, 0, s, A, B, C, M, N, K, lda, ldb, sA, sB, sC, alpha, tm, tn, k_split, part,
-                                   e.bias, e.accum, *e.sq, RowSums{});
-        return;
-    }
+    auto go = [&](auto kernel, const GemmGroup& g, const RowSums& rs) {
+        hipLaunchKernelGGL(kernel, grid, block, 0, s, A, B, C, M, N, K, lda, ldb, sA, sB, sC, alpha, tm, tn, k_split,
+                           part, e.bias, e.accum, g, rs);
+    };
+    // k_gemm<..., STATS, GRP, KSEG, RSUM, SEG> of the transposes that each form takes
     if constexpr (TA && !TB)
         if (e.seg)
         {
-            if (guard)
-                hipLaunchKernelGGL((k_gemm<WM, WN, FM, FN, BK, TA, TB, true, false, false, true>), grid, block, 0, s, A,
-                                   B, C, M, N, K, lda, ldb, sA, sB, sC, alpha, tm, tn, k_split, part, e.bias, e.accum,
-                                   *e.seg);
-            else
-                hipLaunchKernelGGL((k_gemm<WM, WN, FM, FN, BK, TA, TB, false, false, false, true>), grid, block, 0, s,
-                                   A, B, C, M, N, K, lda, ldb, sA, sB, sC, alpha, tm, tn, k_split, part, e.bias,
-                                   e.accum, *e.seg);
+            if (e.by_seq) go(k_gemm<WM, WN, FM, FN, NBUF, TA, TB, false, false, true, false, true>, *e.seg, {});
+            else go(k_gemm<WM, WN, FM, FN, NBUF, TA, TB, false, false, true>, *e.seg, {});
             return;
         }
-    if constexpr (!TA)
-        if (e.grp && e.rs)
+    if constexpr (!TA && TB)
+        if (e.grp && e.by_seq)
         {
-            if (guard)
-                hipLaunchKernelGGL((k_gemm<WM, WN, FM, FN, BK, TA, TB, true, false, true, false, true>), grid, block, 0,
-                                   s, A, B, C, M, N, K, lda, ldb, sA, sB, sC, alpha, tm, tn, k_split, part, e.bias,
-                                   e.accum, *e.grp, *e.rs);
-            else
-                hipLaunchKernelGGL((k_gemm<WM, WN, FM, FN, BK, TA, TB, false, false, true, false, true>), grid, block,
-                                   0, s, A, B, C, M, N, K, lda, ldb, sA, sB, sC, alpha, tm, tn, k_split, part, e.bias,
-                                   e.accum, *e.grp, *e.rs);
+            if (e.rs) go(k_gemm<WM, WN, FM, FN, NBUF, TA, TB, false, true, false, true, true>, *e.grp, *e.rs);
+            else go(k_gemm<WM, WN, FM, FN, NBUF, TA, TB, false, true, false, false, true>, *e.grp, {});
+            return;
+        }
+    if constexpr (!TA && !TB)
+        if (e.by_seq)
+        {
+            go(k_gemm<WM, WN, FM, FN, NBUF, TA, TB, false, false, false, false, true>, *e.sq, {});
             return;
         }
     if constexpr (!TA)
         if (e.grp)
         {
-            if (guard)
-                hipLaunchKernelGGL((k_gemm<WM, WN, FM, FN, BK, TA, TB, true, false, true>), grid, block, 0, s, A, B, C,
-                                   M, N, K, lda, ldb, sA, sB, sC, alpha, tm, tn, k_split, part, e.bias, e.accum,
-                                   *e.grp);
-            else
-                hipLaunchKernelGGL((k_gemm<WM, WN, FM, FN, BK, TA, TB, false, false, true>), grid, block, 0, s, A, B,
-                                   C, M, N, K, lda, ldb, sA, sB, sC, alpha, tm, tn, k_split, part, e.bias, e.accum,
-                                   *e.grp);
+            if (e.rs) go(k_gemm<WM, WN, FM, FN, NBUF, TA, TB, false, true, false, true>, *e.grp, *e.rs);
+            else go(k_gemm<WM, WN, FM, FN, NBUF, TA, TB, false, true>, *e.grp, {});
             return;
         }
-    if (guard)
-        hipLaunchKernelGGL((k_gemm<WM, WN, FM, FN, BK, TA, TB, true>), grid, block, 0, s, A, B, C, M, N, K, lda, ldb,
-                           sA, sB, sC, alpha, tm, tn, k_split, part, e.bias, e.accum, GemmGroup{});
-    else
-        hipLaunchKernelGGL((k_gemm<WM, WN, FM, FN, BK, TA, TB, false>), grid, block, 0, s, A, B, C, M, N, K, lda, ldb,
-                           sA, sB, sC, alpha, tm, tn, k_split, part, e.bias, e.accum, GemmGroup{});
+    go(k_gemm<WM, WN, FM, FN, NBUF, TA, TB>, GemmGroup{}, {});
 }
 
 template <bool TA, bool TB>
 void launch_trans(const Plan& p, const float* A, const float* B, float* C, int M, int N, int K, long lda, long ldb,
                   long sA, long sB, long sC, float alpha, int batch, float* part, hipStream_t s, Epi e)
 {
-    const bool vec_ok = (lda % 4 == 0) && (ldb % 4 == 0) && (sA % 4 == 0) && (sB % 4 == 0) && aligned16(A) &&
-                        aligned16(B);
+    auto go = [&](auto launch) {
+        launch(A, B, C, M, N, K, lda, ldb, sA, sB, sC, alpha, batch, p.splits, p.k_split, part, s, e);
+    };
     switch (p.cfg)
     {
-    case kSkinnyN:
-        launch_cfg<4, 1, 2, 2, 16, TA, TB>(A, B, C, M, N, K, lda, ldb, sA, sB, sC, alpha, batch, vec_ok, p.splits,
-                                           p.k_split, part, s, e);
-        break;
-    case kThinWaves:
-        launch_cfg<4, 1, 1, 2, 16, TA, TB>(A, B, C, M, N, K, lda, ldb, sA, sB, sC, alpha, batch, vec_ok, p.splits,
-                                           p.k_split, part, s, e);
-        break;
-    case kThinWavesM64:
-        launch_cfg<2, 2, 1, 2, 16, TA, TB>(A, B, C, M, N, K, lda, ldb, sA, sB, sC, alpha, batch, vec_ok, p.splits,
-                                           p.k_split, part, s, e);
-        break;
-    case kTall:
-        launch_cfg<4, 2, 2, 2, 16, TA, TB>(A, B, C, M, N, K, lda, ldb, sA, sB, sC, alpha, batch, vec_ok, p.splits,
-                                           p.k_split, part, s, e);
-        break;
-    default:
-        launch_cfg<2, 2, 2, 2, 16, TA, TB>(A, B, C, M, N, K, lda, ldb, sA, sB, sC, alpha, batch, vec_ok, p.splits,
-                                           p.k_split, part, s, e);
-        break;
+    case kSkinnyN: go(launch_cfg<4, 1, 2, 2, 1, TA, TB>); break;
+    case kThinWaves: go(launch_cfg<2, 2, 2, 1, 1, TA, TB>); break;
+    case kThinWavesM64: go(launch_cfg<2, 2, 1, 2, 1, TA, TB>); break;
+    case kTall: go(launch_cfg<4, 2, 2, 2, 2, TA, TB>); break;
+    default: go(launch_cfg<2, 2, 2, 2, 1, TA, TB>); break;
     }
 }
 
@@ -1386,16 +1427,10 @@ extern "C" int nnhip_gemm_colstats(const float* A, const float* B, float* C, siz
     if (!A || !B || !C || !stats) return -1;
     const int m = (int)M, n = (int)N, k = (int)K;
     const int tm = (m + kStatsBM - 1) / kStatsBM, tn = (n + kStatsBN - 1) / kStatsBN;
-    const bool vec = (A_cols % 4 == 0) && (B_cols % 4 == 0) && aligned16(A) && aligned16(B);
-    const bool guard = !vec || (m % kStatsBM) || (n % kStatsBN) || (k % 16);
     const dim3 grid(static_cast<unsigned>(tm * tn), 1, 1), block(512);
-    auto s = static_cast<hipStream_t>(stream);
-    if (guard)
-        hipLaunchKernelGGL((k_gemm<4, 2, 2, 2, 16, false, false, true, true>), grid, block, 0, s, A, B, C, m, n, k,
-                           (long)A_cols, (long)B_cols, 0L, 0L, 0L, 1.0f, tm, tn, k, stats, row_bias, 0, GemmGroup{});
-    else
-        hipLaunchKernelGGL((k_gemm<4, 2, 2, 2, 16, false, false, false, true>), grid, block, 0, s, A, B, C, m, n, k,
-                           (long)A_cols, (long)B_cols, 0L, 0L, 0L, 1.0f, tm, tn, k, stats, row_bias, 0, GemmGroup{});
+    hipLaunchKernelGGL((k_gemm<4, 2, 2, 2, 2, false, false, true>), grid, block, 0, static_cast<hipStream_t>(stream),
+                       A, B, C, m, n, k, (long)A_cols, (long)B_cols, 0L, 0L, 0L, 1.0f, tm, tn, k, stats, row_bias, 0,
+                       GemmGroup{}, RowSums{});
     return launch_status();
 }
 
