@@ -244,7 +244,7 @@ struct SegList
 // merges these instead of reading C once more for them. Needs splits == 1.
 template <int WM, int WN, int FM, int FN, int NBUF, bool TA, bool TB, bool STATS = false, bool GRP = false,
           bool KSEG = false, bool RSUM = false, bool SEG = false>
-__global__ __launch_bounds__(64 * WM * WN, FM * FN == 4 ? 2 : FM * FN == 2 ? 3 : 4) void k_gemm(
+__global__ __launch_bounds__(64 * WM * WN, FM * FN == 4 ? 2 : 3) void k_gemm(
     const float* __restrict__ A, const float* __restrict__ B, float* __restrict__ C, int M, int N, int K, long lda,
     long ldb, long strideA, long strideB, long strideC, float alpha, int tiles_m, int tiles_n, int k_split,
     float* __restrict__ part, const float* __restrict__ bias, int accum, GemmGroup grp, RowSums rs)
@@ -716,60 +716,27 @@ __global__ __launch_bounds__(256) void k_splitk_reduce(const float* __restrict__
     }
 }
 
-// Launch plan for one GEMM: tile configuration and split-K factor.
-enum Cfg { kTall, kSquare, kSkinnyN, kThinWaves, kThinWavesM64 };
-struct Plan
+// What callers are told about a product before it runs: whole tiles for
+// operands by sequence (bm, bn), and the split-K partials that a workspace is
+// sized for and that nnhip_gemm_noalloc's scratch is compared with. Fixed by
+// the shape alone; the launch's own tiles and splits (plan_gemm) stay within.
+struct Terms
 {
-    Cfg cfg;
-    int bm, bn, splits, k_split;
+    int bm, bn, splits;
 };
-
-// Tile choice, from sweeps of the config-3 and config-4 shapes on MI355X.
-// The work is balanced over the 1024 SIMDs first: a 768 x 8192 output makes
-// only 192 tiles of 256 x 128, and any tiling with 64 x 64 per wave leaves
-// either idle CUs or 1.5 waves per SIMD; 32 x 64 per wave (128 x 64 tiles of
-// 4 waves: 768 workgroups, 3 waves on every SIMD) took those products from
-// 69-80 to 87-98 TF/s and the 64-row attention products from 48-61 to 70-85.
-//   * M <= 64: 64 x 128 tiles of 4 waves with 32 x 64 each;
-//   * N <= 64: 256 x 64;
-//   * at least 512 tiles of 256 x 128: 256 x 128 over 8 waves;
-//   * K >= 4096 with a workspace: 256 x 128 (128 x 128 below 128 tiles) with
-//     K split into slices (weight gradients, K = tokens: measured faster than
-//     the thin tiles there);
-//   * otherwise 128 x 64 tiles of 4 waves with 32 x 64 each, K split when the
-//     grid is small and K >= 1024.
-// Split K: slices of >= 256 k for about three workgroups per CU, partial
-// tiles summed in slice order by k_splitk_reduce (deterministic).
-Plan plan_gemm(size_t M, size_t N, size_t K, size_t batch, bool allow_split)
+Terms gemm_terms(size_t M, size_t N, size_t K, size_t batch, bool allow_split)
 {
-    Plan p;
-    p.splits = 1;
-    p.k_split = static_cast<int>(K);
-    auto tiles = [&](int bm, int bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn) * batch; };
-    auto split = [&](size_t t) {
-        size_t want = (768 + t - 1) / t;
-        const size_t max_splits = K / 256;
-        if (want > max_splits) want = max_splits;
+    auto tiles = [&](size_t bm, size_t bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn) * batch; };
+    auto slices = [&](size_t want) {   // whole 32-deep stages a slice
+        if (want > K / 256) want = K / 256;
         if (want > 64) want = 64;
-        if (want > 1)
-        {
-            size_t ks = (K + want - 1) / want;
-            ks = (ks + 31) / 32 * 32;   // whole BK stages per slice
-            p.k_split = static_cast<int>(ks);
-            p.splits = static_cast<int>((K + ks - 1) / ks);
-        }
+        if (want <= 1) return 1;
+        const size_t ks = ((K + want - 1) / want + 31) / 32 * 32;
+        return static_cast<int>((K + ks - 1) / ks);
     };
-    // Mid-sized outputs with K >= 2048: split K so that the workgroups make whole
-    // rounds of 3 per CU (768 on MI355X); the first of 256x128, 128x128, 128x64
-    // whose split leaves >= 1024 of K per slice (measured on the config-3/4
-    // shapes: 6144x768 K8192 NT 110 -> 123, 768x3072 K8192 NT 105 -> 115,
-    // 768x8192 K3072 NN 121 -> 124 TFLOP/s; round counts that are not whole lose
-    // the fraction).
+    const size_t round = 3 * static_cast<size_t>(device_cus());
+    const int bms[3] = {256, 128, 128}, bns[3] = {128, 128, 64};
     if (M > 64 && N > 64 && allow_split && K >= 2048 && tiles(256, 128) < 512)
-    {
-        const size_t round = 3 * static_cast<size_t>(device_cus());
-        const Cfg cs[3] = {kTall, kSquare, kThinWaves};
-        const int bms[3] = {256, 128, 128}, bns[3] = {128, 128, 64};
         for (int i = 0; i < 3; ++i)
         {
             const size_t t = tiles(bms[i], bns[i]);
@@ -777,79 +744,111 @@ Plan plan_gemm(size_t M, size_t N, size_t K, size_t batch, bool allow_split)
             while (s <= 64 && (t * s) % round != 0) ++s;
             if (s > 64) continue;
             const size_t ks = ((K + s - 1) / s + 31) / 32 * 32;
-            if (ks < 1024) continue;
-            p.cfg = cs[i];
-            p.bm = bms[i];
-            p.bn = bns[i];
-            p.k_split = static_cast<int>(ks);
-            p.splits = static_cast<int>((K + ks - 1) / ks);
-            return p;
+            if (ks >= 1024) return {bms[i], bns[i], static_cast<int>((K + ks - 1) / ks)};
         }
-    }
-    if (M <= 64) { p.cfg = kThinWavesM64; p.bm = 64; p.bn = 128; }
-    else if (N <= 64) { p.cfg = kSkinnyN; p.bm = 256; p.bn = 64; }
+    Terms p{128, 64, 1};
+    if (M <= 64) p = {64, 128, 1};
+    else if (N <= 64) p = {256, 64, 1};
     else if (tiles(256, 128) >= 512)
     {
-        p.cfg = kTall;
-        p.bm = 256;
-        p.bn = 128;
-        // Under 4 resident rounds of 256x128 tiles the last, partial round
-        // costs a whole round: take smaller tiles when their whole rounds win
-        // clearly (per-tile efficiency 1 : 0.985 : 0.94 measured on the config-3/4
-        // shapes; 8192x2304 K768: 576 tiles of 256x128, 94 -> 120 TFLOP/s as
-        // 2304 of 128x64). Grids of >= 4 rounds (the lm_head product) keep 256x128.
-        const double round = 3.0 * device_cus();
-        if (static_cast<double>(tiles(256, 128)) < 4.0 * round)
+        p = {256, 128, 1};
+        if (static_cast<double>(tiles(256, 128)) < 4.0 * static_cast<double>(round))
         {
             auto est = [&](size_t t, double eff) {
-                const double r = static_cast<double>(t) / round;
+                const double r = static_cast<double>(t) / static_cast<double>(round);
                 return r / std::ceil(r) * eff;
             };
             const double eT = est(tiles(256, 128), 1.0), eS = est(tiles(128, 128), 0.985),
                          eN = est(tiles(128, 64), 0.94);
-            if (eN > eT + 0.05 && eN >= eS) { p.cfg = kThinWaves; p.bm = 128; p.bn = 64; }
-            else if (eS > eT + 0.05) { p.cfg = kSquare; p.bm = 128; p.bn = 128; }
+            if (eN > eT + 0.05 && eN >= eS) p = {128, 64, 1};
+            else if (eS > eT + 0.05) p = {128, 128, 1};
         }
     }
     else if (allow_split && K >= 4096)
     {
-        p.cfg = kTall;
-        p.bm = 256;
-        p.bn = 128;
-        if (tiles(128, 128) < 128)
-        {
-            // Small outputs from long K (the 768 x 768 weight gradients over 8192
-            // tokens, alone or as the q, k, v group): 128 x 64 tiles split to
-            // about 1728 workgroups (q, k, v group 101 -> 111 TFLOP/s, the single
-            // one unchanged at 95-97, against 128 x 128 tiles split to 768).
-            p.cfg = kThinWaves;
-            p.bm = 128;
-            p.bn = 64;
-            const size_t t = tiles(128, 64);
-            size_t want = (1728 + t - 1) / t;
-            if (want > K / 256) want = K / 256;
-            if (want > 64) want = 64;
-            if (want > 1)
-            {
-                const size_t ks = ((K + want - 1) / want + 31) / 32 * 32;
-                p.k_split = static_cast<int>(ks);
-                p.splits = static_cast<int>((K + ks - 1) / ks);
-            }
-            return p;
-        }
-        if (tiles(256, 128) < 128)
-        {
-            p.cfg = kSquare;
-            p.bm = 128;
-            p.bn = 128;
-        }
-        split(tiles(p.bm, p.bn));
+        if (tiles(128, 128) < 128) return {128, 64, slices((1728 + tiles(128, 64) - 1) / tiles(128, 64))};
+        p = tiles(256, 128) < 128 ? Terms{128, 128, 1} : Terms{256, 128, 1};
+        p.splits = slices((768 + tiles(p.bm, p.bn) - 1) / tiles(p.bm, p.bn));
         return p;
     }
-    else { p.cfg = kThinWaves; p.bm = 128; p.bn = 64; }
     const size_t t = tiles(p.bm, p.bn);
-    if (allow_split && t < 512 && K >= 1024) split(t);
+    if (allow_split && t < 512 && K >= 1024) p.splits = slices((768 + t - 1) / t);
     return p;
+}
+size_t partial_bytes(size_t M, size_t N, size_t batch, int splits)
+{
+    // (split-K partial tiles, and the slices' row sums of nnhip_gemm_group_acc)
+    return splits > 1 ? static_cast<size_t>(splits) * batch * (M * N + M) * sizeof(float) : 0;
+}
+
+// Launch plan for one GEMM: the tile and the split of K.
+enum Cfg { kTall, kThin, kSmall };
+struct Plan
+{
+    Cfg cfg;
+    int splits, k_split;
+};
+// The tiles, each with what a CU takes for one 32-deep stage of n of its
+// workgroups at once (us; n up to what its LDS and registers let it hold) and
+// a launch's fixed part, measured on MI355X over 62 products of 128..32000
+// with every tile and split. In whole products: 256 x 128 at 1 workgroup a CU
+// 4096^3 220 TFLOP/s against 183 of 128 x 128 and 166 of 128 x 64 tiles;
+// 64 x 64 tiles 768 x 4096 x 768 129 against 108 (128 x 64) and 114 (256 x 128
+// split in two), and 512 x 128 x 128 in 6.4 us against 8.9. Also measured and
+// nowhere the best by more than 3 %: 128 x 128, 256 x 64, 64 x 128.
+struct Tile
+{
+    int bm, bn, held;
+    double stage[3], fixed;
+};
+constexpr Tile kTiles[3] = {{256, 128, 1, {2.35, 0, 0}, 6.0},
+                            {128, 64, 3, {1.22, 1.65, 2.45}, 5.0},
+                            {64, 64, 3, {0.62, 0.95, 1.38}, 4.0}};
+
+// The tile and split with the least estimated time: the stages of the CU with
+// the most workgroups, the stores, and for split K the partials' sum (3 us and
+// its bytes at 5.5 TB/s). The estimate picks within 2 % of the best measured
+// one on average over those 62. Partials take at most `budget` bytes; K below
+// 1024 is never split (a product and its heads-layout form sum alike there).
+constexpr size_t kSplitBudget = NNHIP_GEMM_NOALLOC_SCRATCH_BYTES;
+Plan plan_gemm(size_t M, size_t N, size_t K, size_t batch, size_t budget)
+{
+    static constexpr int kSplits[] = {1, 2, 3, 4, 5, 6, 8, 10, 12, 16, 20, 24, 32, 48, 64};
+    Plan best{kThin, 1, static_cast<int>(K)};
+    double least = 1e300;
+    const double out_mb = static_cast<double>(M) * static_cast<double>(N) * static_cast<double>(batch) * 4e-6;
+    for (const int want : kSplits)
+    {
+        const size_t ks = want == 1 ? K : ((K + want - 1) / want + 31) / 32 * 32;
+        if (want > 1 && (K < 1024 || ks < 128 || (K + ks - 1) / ks != static_cast<size_t>(want) ||
+                         partial_bytes(M, N, batch, want) > budget))
+            continue;
+        const double stages = static_cast<double>((ks + BK - 1) / BK);
+        const double tail = want > 1 ? 3.0 + out_mb * (want + 1) / 5.5 : 0.0;
+        for (int c = 0; c < 3; ++c)
+        {
+            const Tile& t = kTiles[c];
+            const double wgs = static_cast<double>((M + t.bm - 1) / t.bm) *
+                               static_cast<double>((N + t.bn - 1) / t.bn) * static_cast<double>(batch) * want;
+            const double n = std::ceil(wgs / device_cus()), rounds = std::floor(n / t.held);
+            const int rest = static_cast<int>(n - rounds * t.held);
+            double us = stages * (rounds * t.stage[t.held - 1] + (rest ? t.stage[rest - 1] : 0.0));
+            if (rounds >= 2) us *= 0.93;   // (uneven ends overlap)
+            us += t.fixed + tail + out_mb * want / 12.0;
+            if (us < least)
+            {
+                least = us;
+                best = {static_cast<Cfg>(c), want, static_cast<int>(ks)};
+            }
+        }
+    }
+    return best;
+}
+// The bytes of partials that the plan of a product may take given a workspace.
+size_t split_budget(size_t M, size_t N, size_t K, size_t batch)
+{
+    const size_t told = partial_bytes(M, N, batch, gemm_terms(M, N, K, batch, true).splits);
+    return told > kSplitBudget ? told : kSplitBudget;
 }
 
 struct Epi
@@ -915,11 +914,9 @@ void launch_trans(const Plan& p, const float* A, const float* B, float* C, int M
     };
     switch (p.cfg)
     {
-    case kSkinnyN: go(launch_cfg<4, 1, 2, 2, 1, TA, TB>); break;
-    case kThinWaves: go(launch_cfg<2, 2, 2, 1, 1, TA, TB>); break;
-    case kThinWavesM64: go(launch_cfg<2, 2, 1, 2, 1, TA, TB>); break;
     case kTall: go(launch_cfg<4, 2, 2, 2, 2, TA, TB>); break;
-    default: go(launch_cfg<2, 2, 2, 2, 1, TA, TB>); break;
+    case kThin: go(launch_cfg<2, 2, 2, 1, 1, TA, TB>); break;
+    case kSmall: go(launch_cfg<2, 2, 1, 1, 2, TA, TB>); break;
     }
 }
 
@@ -1344,22 +1341,28 @@ int gemm_dispatch(const float* A, const float* B, float* C, size_t M, size_t N, 
     if (int rc = 0; !e.grp && !e.seg && !e.by_seq &&
                     try_gemv(A, B, C, M, N, K, lda, ldb, sA, sB, sC, tA, tB, alpha, batch, s, e, rc))
         return rc;
-    Plan p = plan_gemm(M, N, K, batch, workspace != nullptr);
-    if (p.splits > 1 && static_cast<size_t>(p.splits) * batch * (M * N + (e.rs ? M : 0)) * sizeof(float) > ws_bytes)
-        p = plan_gemm(M, N, K, batch, false);
+    auto need = [&](int splits) {
+        return splits > 1 ? static_cast<size_t>(splits) * batch * (M * N + (e.rs ? M : 0)) * sizeof(float) : 0;
+    };
+    Plan p = plan_gemm(M, N, K, batch, workspace ? split_budget(M, N, K, batch) : 0);
+    if (need(p.splits) > ws_bytes) p = plan_gemm(M, N, K, batch, workspace ? ws_bytes : 0);
     if (e.by_seq)
     {
+        Terms w = gemm_terms(M, N, K, batch, workspace != nullptr);
+        if (need(w.splits) > ws_bytes) w = gemm_terms(M, N, K, batch, false);
         // whole tiles, 16-byte loads, and no tile or stage across two sequences
         const GemmGroup& g = e.grp ? *e.grp : e.seg ? *e.seg : *e.sq;
-        const bool whole = M % p.bm == 0 && N % p.bn == 0 && K % 16 == 0 && p.k_split % 16 == 0 && lda % 4 == 0 &&
-                           ldb % 4 == 0 && sA % 4 == 0 && sB % 4 == 0 && aligned16(A) && aligned16(B);
+        const bool whole = M % w.bm == 0 && N % w.bn == 0 && K % 16 == 0 && lda % 4 == 0 && ldb % 4 == 0 &&
+                           sA % 4 == 0 && sB % 4 == 0 && aligned16(A) && aligned16(B);
         if (!whole) return -7;
         const int members = e.grp ? static_cast<int>(batch / g.nb) : 1;
         for (int i = 0; i < members && i < kGroupMax; ++i)
         {
             if (g.aT[i] < 0 || g.bT[i] < 0 || g.aS[i] % 4 != 0 || g.bS[i] % 4 != 0) return -7;
             if (g.aT[i] && (tA || g.aT[i] % 16 != 0 || g.aS[i] < g.aT[i])) return -7;
-            if (g.bT[i] && (g.bT[i] % (tB ? 16 : p.bn) != 0 || g.bS[i] < g.bT[i])) return -7;
+            if (g.bT[i] && (g.bT[i] % (tB ? 16 : w.bn) != 0 || g.bS[i] < g.bT[i])) return -7;
+            // (the tile in use may be the wider one)
+            if (!tB && g.bT[i] % kTiles[p.cfg].bn != 0) p.cfg = kThin;
         }
     }
     float* part = p.splits > 1 ? static_cast<float*>(workspace) : nullptr;
@@ -1402,8 +1405,9 @@ int gemm_dispatch(const float* A, const float* B, float* C, size_t M, size_t N, 
 constexpr int kStatsBM = 256, kStatsBN = 128;
 bool colstats_ok(size_t M, size_t N, size_t K, int tA, int tB)
 {
-    return !tA && !tB && M > 0 && N > 0 && K > 0 && M <= 0x7fffffff && N <= 0x7fffffff && K <= 0x7fffffff &&
-           plan_gemm(M, N, K, 1, false).cfg == kTall;
+    if (tA || tB || M == 0 || N == 0 || K == 0 || M > 0x7fffffff || N > 0x7fffffff || K > 0x7fffffff) return false;
+    const Terms t = gemm_terms(M, N, K, 1, false);
+    return t.bm == kStatsBM && t.bn == kStatsBN;
 }
 
 } // namespace
@@ -1436,9 +1440,9 @@ extern "C" int nnhip_gemm_colstats(const float* A, const float* B, float* C, siz
 
 extern "C" size_t nnhip_gemm_workspace_bytes(size_t M, size_t N, size_t K, size_t batch)
 {
-    // (split-K partial tiles, and the slices' row sums of nnhip_gemm_group_acc)
-    const Plan p = plan_gemm(M, N, K, batch, true);
-    return p.splits > 1 ? static_cast<size_t>(p.splits) * batch * (M * N + M) * sizeof(float) : 0;
+    const size_t told = partial_bytes(M, N, batch, gemm_terms(M, N, K, batch, true).splits);
+    const size_t used = partial_bytes(M, N, batch, plan_gemm(M, N, K, batch, split_budget(M, N, K, batch)).splits);
+    return told > used ? told : used;
 }
 
 extern "C" int nnhip_gemm(const float* A, const float* B, float* C, size_t A_rows, size_t A_cols, size_t B_rows,
