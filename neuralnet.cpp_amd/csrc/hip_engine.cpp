@@ -2737,7 +2737,7 @@ Result<Tensor> HipEngine::batched_matmul_softmax_apply(const Tensor& A, const Te
         NN_TRY(o, alloc_(batch * d.M, V.cols()));
         NN_TRY(cells, mask_cells_buf_(mask, d.M, d.N));
         // A recorded output also keeps the forward's scores for the backward
-        // (one 32 x 32 block per cell, so M and N whole tiles), while all
+        // (one 32 x 32 block per cell, the last ones padded), while all
         // records together hold at most score_budget_ bytes of them. The
         // blocks only save work: when they cannot be had, the backward forms
         // the scores itself.
@@ -2749,9 +2749,10 @@ Result<Tensor> HipEngine::batched_matmul_softmax_apply(const Tensor& A, const Te
             if (ptwo_.size() >= kKeep) ptwo_.erase(ptwo_.begin());
             std::size_t held = 0;
             for (const TwoPassOut& r : ptwo_) held += r.S.size() * sizeof(float);
-            if (d.M % 32 == 0 && d.N % 32 == 0 && held + batch * d.M * d.N * sizeof(float) <= score_budget_)
+            const std::size_t Mp = (d.M + 31) / 32 * 32, Np = (d.N + 31) / 32 * 32;
+            if (held + batch * Mp * Np * sizeof(float) <= score_budget_)
             {
-                auto t = alloc_(batch * d.M, d.N);
+                auto t = alloc_(batch * Mp, Np);
                 if (t) S = *t;
             }
         }

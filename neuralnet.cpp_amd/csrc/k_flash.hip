@@ -1,4 +1,5 @@
-// k_flash.hip — one-pass attention chains on the fp32 matrix cores.
+// k_flash.hip — one-pass attention chains on the matrix cores: float32 split into bf16 parts (split_bf16.hpp), with
+// the float32 chains where those do not hold.
 //
 // The reference's two-pass attention is a chain of engine primitives
 // (compute_layer.hpp:1196-1221 forward, :1304-1327 backward):
@@ -43,7 +44,11 @@
 // contracts over tokens drow(r,0), drow(r,1). Contraction dims are permuted so
 // LDS reads are vectors: score step kk reads dim kk + KP/2*h (4 steps per
 // 16-byte read); output tile u row i holds dim DU*i + u (one 8-byte read feeds
-// both tiles when DU = 2).
+// both tiles when DU = 2). The split chains' operands are described where they
+// are built (STile, VTile). Measured on MI355X against the float32 chains
+// alone, forward / key-line pass / dQ pass in us: causal 128 heads T 512 64 ->
+// 51, 99 -> 78, 40 -> 37; document rows 96 heads T 2048 246 -> 172, 381 -> 263,
+// 128 -> 112; ALiBi 48 heads T 1024 108 -> 83, 139 -> 103, 41 -> 41.
 #include "flash.hpp"
 
 #include <algorithm>
@@ -52,6 +57,7 @@
 
 #include "common.hpp"
 #include "nnhip_kernels.h"
+#include "split_bf16.hpp"
 
 namespace nnhip
 {
@@ -308,24 +314,13 @@ __device__ __forceinline__ void mask_row16(const MRow& x, int N, int jbase, int 
 }
 
 // Score chain: D[token drow(r,h)][line token c] = sum_k tile[c][k] * reg[k] over KP dims.
-// Scheduling fence after a chain's LDS reads when PRE: only VALU, SALU and
-// transcendental instructions may move across it, so the reads are all issued
-// before the first MFMA and the chain runs without waiting on LDS (costs the
-// registers of the whole A operand).
-template <bool PRE>
-__device__ __forceinline__ void operands_first()
-{
-    if constexpr (PRE) __builtin_amdgcn_sched_barrier(0x0406);
-}
-
-template <int KP, bool PRE = false>
+template <int KP>
 __device__ __forceinline__ f32x16 score_chain(const float (*tile)[KP + 4], const float* reg, int h, int c)
 {
     constexpr int KH = KP / 2;
     float4 a[KH / 4];
 #pragma unroll
     for (int q4 = 0; q4 < KH / 4; ++q4) a[q4] = *reinterpret_cast<const float4*>(&tile[c][KH * h + 4 * q4]);
-    operands_first<PRE>();
     f32x16 s = zero16();
 #pragma unroll
     for (int q4 = 0; q4 < KH / 4; ++q4)
@@ -339,7 +334,7 @@ __device__ __forceinline__ f32x16 score_chain(const float (*tile)[KP + 4], const
 }
 
 // acc[u] += tile^T (dims DU*c + u, tokens drow(r,h)) x w (tokens drow(r,h), line token c).
-template <int DP, bool PRE = false>
+template <int DP>
 __device__ __forceinline__ void value_chain(const float (*tile)[DP + 4], const float* w, int h, int c, f32x16* acc)
 {
     constexpr int DU = DP / 32;
@@ -348,8 +343,7 @@ __device__ __forceinline__ void value_chain(const float (*tile)[DP + 4], const f
         float2 a[16];
 #pragma unroll
         for (int r = 0; r < 16; ++r) a[r] = *reinterpret_cast<const float2*>(&tile[drow(r, h)][2 * c]);
-        operands_first<PRE>();
-#pragma unroll
+    #pragma unroll
         for (int r = 0; r < 16; ++r)
         {
             acc[0] = mfma(a[r].x, w[r], acc[0]);
@@ -361,8 +355,7 @@ __device__ __forceinline__ void value_chain(const float (*tile)[DP + 4], const f
         float a[16];
 #pragma unroll
         for (int r = 0; r < 16; ++r) a[r] = tile[drow(r, h)][c];
-        operands_first<PRE>();
-#pragma unroll
+    #pragma unroll
         for (int r = 0; r < 16; ++r) acc[0] = mfma(a[r], w[r], acc[0]);
     }
 }
@@ -405,6 +398,190 @@ __device__ __forceinline__ void line_operand(const float* base, int dims, int T,
         const int d = kk + KH * h;
         reg[kk] = (t < T && d < dims) ? base[(long)d * T + tc] : 0.0f;
     }
+}
+
+// ── the same chains on the bf16 matrix cores (split_bf16.hpp) ───────────────
+// A tile's floats are split when they are staged, a line's operand once, and
+// the weights of a cell in registers. Both tile forms hold 8 elements of the
+// contraction (an MFMA operand's share of a lane) in 16 bytes:
+//   score form  [token][dim], the chain over dims;
+//   value form  [dim][token], the chain over tokens. A lane's weights are its
+//     score registers 8 s .. 8 s + 7 of step s, tokens 16 s + 4 h + 0..3 and
+//     + 8..11: the octet 2 s + h holds those tokens, so weights never move
+//     between lanes. Row u 32 + i holds dim DU i + u (the outputs' order).
+// Rows of 64 or 128 bytes, octets swapped so that 16 neighbouring rows' same
+// octet covers the LDS banks once. A cell of KP = DP = 64 is 48 MFMAs of 32
+// cycles forward where the float32 chains take 64 of 64.
+typedef bf16x8 Parts[3];
+
+template <int KP>
+struct STile
+{
+    static constexpr int OCT = KP / 8;
+    typedef bf16x8 Lds[3][32 * OCT];
+    floatx8 r;
+    static __device__ __forceinline__ int slot(int tok, int o)
+    {
+        return tok * OCT + (o ^ (OCT == 8 ? (tok >> 1) & 7 : (tok >> 2) & 3));
+    }
+    static __device__ __forceinline__ bool mine() { return threadIdx.x < 32 * OCT; }
+    // from a (dims, T) [dim][token] array: thread t holds token t % 32, dims 8 (t / 32) ..
+    __device__ __forceinline__ void load(const float* base, int dims, int T, int t0)
+    {
+        if (!mine()) return;
+        const Rsrc rs = rsrc(base, (long)dims * T);
+        const int t = t0 + static_cast<int>(threadIdx.x & 31), d0 = 8 * static_cast<int>(threadIdx.x >> 5);
+#pragma unroll
+        for (int e = 0; e < 8; ++e)   // dims past the array fall past the resource by themselves
+            r[e] = bload(rs, oob_if_neg(4u * static_cast<unsigned>((d0 + e) * T + t), T - 1 - t));
+    }
+    __device__ __forceinline__ void store(const SplitUnits& su, Lds& l) const
+    {
+        if (!mine()) return;
+        const int o = slot(threadIdx.x & 31, threadIdx.x >> 5);
+        split3(su, r, l[0][o], l[1][o], l[2][o]);
+    }
+};
+
+template <int DP>
+struct VTile
+{
+    typedef bf16x8 Lds[3][DP * 4];
+    floatx8 r;
+    static __device__ __forceinline__ int slot(int row, int o) { return row * 4 + (o ^ ((row >> 2) & 3)); }
+    static __device__ __forceinline__ int row_of(int d) { return DP == 64 ? (d & 1) * 32 + (d >> 1) : d; }
+    static __device__ __forceinline__ bool mine() { return threadIdx.x < 4 * DP; }
+    // first token of octet o = 2 s + h: tokens 16 s + 4 h + 0..3 and + 8..11
+    static __device__ __forceinline__ int tok0(int o) { return 16 * (o >> 1) + 4 * (o & 1); }
+    // from a (dims, T) [dim][token] array: thread t holds dim t / 4, octet t % 4
+    __device__ __forceinline__ void load(const float* base, int dims, int T, int t0)
+    {
+        if (!mine()) return;
+        const Rsrc rs = rsrc(base, (long)dims * T);
+        const int d = threadIdx.x >> 2, t = t0 + tok0(threadIdx.x & 3);
+        if (t0 + 32 <= T)
+        {
+            const float4 x = bload4(rs, 4u * static_cast<unsigned>(d * T + t)),
+                         y = bload4(rs, 4u * static_cast<unsigned>(d * T + t + 8));
+            r = floatx8{x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};
+        }
+        else
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+            {
+                const int te = t + (e < 4 ? e : e + 4);
+                r[e] = bload(rs, oob_if_neg(4u * static_cast<unsigned>(d * T + te), T - 1 - te));
+            }
+    }
+    __device__ __forceinline__ void store(const SplitUnits& su, Lds& l) const
+    {
+        if (!mine()) return;
+        const int o = slot(row_of(threadIdx.x >> 2), threadIdx.x & 3);
+        split3(su, r, l[0][o], l[1][o], l[2][o]);
+    }
+    // from a (T, ld) [token][dim] array (dims < ncols): thread t holds dim t % DP, octet t / DP
+    __device__ __forceinline__ void load_rows(const float* base, int ld, int ncols, int T, int t0)
+    {
+        if (!mine()) return;
+        const Rsrc rs = rsrc(base, (long)T * ld);
+        const int d = threadIdx.x % DP, t = t0 + tok0(threadIdx.x / DP);
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+        {
+            const int te = t + (e < 4 ? e : e + 4);
+            r[e] = bload(rs, oob_if_neg(4u * static_cast<unsigned>(te * ld + d), (T - 1 - te) | (ncols - 1 - d)));
+        }
+    }
+    __device__ __forceinline__ void store_rows(const SplitUnits& su, Lds& l) const
+    {
+        if (!mine()) return;
+        const int o = slot(row_of(threadIdx.x % DP), threadIdx.x / DP);
+        split3(su, r, l[0][o], l[1][o], l[2][o]);
+    }
+};
+
+// Per-lane B operand of a score chain: step s holds dims 16 s + 8 h + 0..7 of token t of a (dims, T) array.
+template <int KP>
+__device__ __forceinline__ void line_parts(const SplitUnits& su, const float* base, int dims, int T, int t, int h,
+                                           Parts* p)
+{
+    const Rsrc rs = rsrc(base, (long)dims * T);
+    floatx8 x[KP / 16];
+#pragma unroll
+    for (int s = 0; s < KP / 16; ++s)
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+            x[s][e] = bload(rs, oob_if_neg(4u * static_cast<unsigned>((16 * s + 8 * h + e) * T + t), T - 1 - t));
+#pragma unroll
+    for (int s = 0; s < KP / 16; ++s) split3(su, x[s], p[s][0], p[s][1], p[s][2]);
+}
+
+__device__ __forceinline__ f32x16 mfma_b(bf16x8 a, bf16x8 b, f32x16 c)
+{
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+}
+
+// D[token drow(r,h)][line token c] = 2^48 sum_k tile[c][k] * line[k] over KP dims.
+template <int KP>
+__device__ __forceinline__ f32x16 score_parts(const typename STile<KP>::Lds& tile, const Parts* line, int h, int c)
+{
+    f32x16 s = zero16(), t = zero16();
+#pragma unroll
+    for (int k = 0; k < KP / 16; ++k)
+    {
+        const int o = STile<KP>::slot(c, 2 * k + h);
+        const bf16x8 ah = tile[0][o], am = tile[1][o], al = tile[2][o];
+        s = mfma_b(ah, line[k][0], s);
+        t = mfma_b(ah, line[k][2], t);
+        t = mfma_b(al, line[k][0], t);
+        t = mfma_b(am, line[k][1], t);
+        t = mfma_b(ah, line[k][1], t);
+        t = mfma_b(am, line[k][0], t);
+    }
+    return s + t;
+}
+
+// The parts of a cell's 16 weights of a lane (scaled by 2^24 already).
+__device__ __forceinline__ void weight_parts(const SplitUnits& su, const float* w, Parts* p)
+{
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+    {
+        floatx8 x;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = w[8 * s + e];
+        split3_scaled(su, x, p[s][0], p[s][1], p[s][2]);
+    }
+}
+
+// acc[u] += 2^48 tile (dims DU*c + u, tokens) x w (tokens, line token c), small products first.
+template <int DP>
+__device__ __forceinline__ void value_parts(const typename VTile<DP>::Lds& tile, const Parts* w, int h, int c,
+                                            f32x16* acc)
+{
+    constexpr int DU = DP / 32;
+    constexpr int pa[6] = {2, 0, 1, 1, 0, 0}, pb[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+    {
+        bf16x8 a[DU][3];
+#pragma unroll
+        for (int u = 0; u < DU; ++u)
+#pragma unroll
+            for (int p = 0; p < 3; ++p) a[u][p] = tile[p][VTile<DP>::slot(32 * u + c, 2 * s + h)];
+#pragma unroll
+        for (int t = 0; t < 6; ++t)
+#pragma unroll
+            for (int u = 0; u < DU; ++u) acc[u] = mfma_b(a[u][pa[t]], w[s][pb[t]], acc[u]);
+    }
+}
+
+// Not zero when one of x's values is not finite.
+__device__ __forceinline__ float not_finite(const f32x16& x, float sum)
+{
+#pragma unroll
+    for (int r = 0; r < 16; ++r) sum = __builtin_fmaf(x[r], 0.0f, sum);
+    return sum;
 }
 
 // ── forward: m, l and (WITH_O) O over query lines ──────────────────────────
@@ -475,10 +652,19 @@ __device__ __forceinline__ void fwd_store(const FlashFwdArgs& a, const FlashGeo&
 // alpha * dot + mask, -inf for keys past N. Returns the cell's row maximum.
 template <bool FULL, bool MASKED>
 __device__ __forceinline__ float cell_scores(const f32x16& s, float alpha, const MRow& mrow, int N, int jbase, int h,
-                                             float* x)
+                                             float* x, const float* held = nullptr)
 {
     float mv[16];
-    if constexpr (MASKED) mask_row16(mrow, N, jbase, h, mv);
+    if constexpr (MASKED)
+    {
+        if (held)
+        {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) mv[r] = held[r];
+        }
+        else
+            mask_row16(mrow, N, jbase, h, mv);
+    }
 #pragma unroll
     for (int r = 0; r < 16; ++r)
     {
@@ -497,124 +683,105 @@ __device__ __forceinline__ float cell_scores(const f32x16& s, float alpha, const
 }
 
 // Forward workgroup: 4 waves on 4 consecutive query lines (32 queries each)
-// walking the non-empty cells of their range CPS (1 or 2) at a time. A step
-// stages the key and value tiles of its cells in LDS (double-buffered, one
-// barrier per step); each wave computes the scores of its active cells,
-// updates its online max / sum once per step (one cross-lane max, one
-// rescale, skipped when no row maximum moved) and accumulates the weighted
-// values.
-template <int KP, int DP, bool WITH_O, bool VDM, int CPS>
-__global__ __launch_bounds__(64 * kWaves, CPS == 1 ? 3 : 2) void k_flash_fwd(FlashFwdSet t, FlashGeo g)
+// walking the non-empty cells of their range. A step stages a cell's key and
+// value tiles in LDS (double-buffered, one barrier per step); each wave
+// computes the scores of its active cells, updates its online max / sum (one
+// cross-lane max, one rescale, skipped when no row maximum moved) and
+// accumulates the weighted values.
+//
+// fwd_split runs the chains on the bf16 matrix cores; what bounds it is those
+// (1536 cycles a cell and wave) beside about 250 vector instructions a cell
+// (scale, mask, max, exp2, and the weights' split), two waves a SIMD covering
+// each other: 48 KB of LDS and 2 workgroups a CU. A workgroup whose results
+// are not all finite, or whose scores are not in a row that has found no
+// weight yet (past the scaled range they are -inf as masked ones are), runs
+// its lines again with fwd_f32, the float32 chains, which take infinities and
+// NaN as they come.
+template <int KP, int DP, bool WITH_O>
+struct FwdLds
+{
+    typename STile<KP>::Lds k[2];
+    typename VTile<WITH_O ? DP : 32>::Lds v[WITH_O ? 2 : 1];
+};
+template <int KP, int DP, bool WITH_O>
+struct FwdLdsF32
+{
+    float k[2][32][KP + 4];
+    float v[WITH_O ? 2 : 1][WITH_O ? 32 : 1][DP + 4];
+};
+
+template <int KP, int DP, bool WITH_O, bool VDM, bool SST>
+__device__ __forceinline__ bool fwd_split(const FlashFwdArgs& a, const FlashGeo& g, const Item& it,
+                                          const LineWork& lw, unsigned long long any, FwdLds<KP, DP, WITH_O>& L)
 {
     constexpr int DU = DP / 32;
-    __shared__ __align__(16) float Ks[2][CPS][32][KP + 4];
-    __shared__ __align__(16) float Vs[WITH_O ? 2 : 1][WITH_O ? CPS : 1][WITH_O ? 32 : 1][DP + 4];
-    __shared__ unsigned long long nz_s[kWaves];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, h = lane >> 5, c = lane & 31;
-    const Item it = item_of(g);
-    const FlashFwdArgs a = row_args(t, g, it.b);
     const int line = it.grp * kWaves + wave, qi = line * 32 + c;
-    const LineWork lw = line_work(g, true, it.b, line, it.rg);
-    if (lane == 0) nz_s[wave] = lw.nz;
-    __syncthreads();
-    const unsigned long long any = nz_s[0] | nz_s[1] | nz_s[2] | nz_s[3];
-
-    float mrun = kLowest, lrun = 0.0f;
+    const SplitUnits su;
+    float mrun = kLowest, lrun = 0.0f, bad = 0.0f;
     f32x16 o[DU];
 #pragma unroll
     for (int u = 0; u < DU; ++u) o[u] = zero16();
     if (any)
     {
         const int cell0 = it.rg * g.R;
-        const float* Qb = a.Q + (long)it.b * a.K * g.M;
         const float* Kb = a.Kt + (long)it.b * a.K * g.N;
         const float* Vb = WITH_O ? a.V + (long)it.b * g.N * a.D : nullptr;
-        TTile<KP> kt[CPS];
-        std::conditional_t<VDM, TTile<DP>, RTile<DP>> vt[CPS];   // V (D, N) or (N, D), staged [key][dim]
-        unsigned long long rest = any;
-        auto pop = [&]() {
-            if (!rest) return -1;
-            const int b = __builtin_ctzll(rest);
-            rest &= rest - 1;
-            return b;
+        STile<KP> kt;
+        VTile<DP> vt;
+        unsigned long long rest = any & (any - 1);
+        auto load = [&](int cell) {
+            kt.load(Kb, a.K, g.N, 32 * (cell0 + cell));
+            if constexpr (WITH_O && VDM) vt.load(Vb, a.D, g.N, 32 * (cell0 + cell));
+            if constexpr (WITH_O && !VDM) vt.load_rows(Vb, a.D, a.D, g.N, 32 * (cell0 + cell));
         };
-        auto load = [&](int c0, int c1) {
-            const int cc[2] = {c0, c1};
-#pragma unroll
-            for (int t = 0; t < CPS; ++t)
-                if (cc[t] >= 0)
-                {
-                    kt[t].load(Kb, a.K, g.N, 32 * (cell0 + cc[t]), threadIdx.x);
-                    if constexpr (WITH_O && VDM) vt[t].load(Vb, a.D, g.N, 32 * (cell0 + cc[t]), threadIdx.x);
-                    if constexpr (WITH_O && !VDM) vt[t].load(Vb, a.D, a.D, g.N, 32 * (cell0 + cc[t]), threadIdx.x);
-                }
+        auto store = [&](int buf) {
+            kt.store(su, L.k[buf]);
+            if constexpr (WITH_O && VDM) vt.store(su, L.v[buf]);
+            if constexpr (WITH_O && !VDM) vt.store_rows(su, L.v[buf]);
         };
-        auto store = [&](int buf, int c0, int c1) {
-            const int cc[2] = {c0, c1};
-#pragma unroll
-            for (int t = 0; t < CPS; ++t)
-                if (cc[t] >= 0)
-                {
-                    kt[t].store(Ks[buf][t], threadIdx.x);
-                    if constexpr (WITH_O) vt[t].store(Vs[buf][t], threadIdx.x);
-                }
-        };
-        int c0 = pop(), c1 = CPS == 2 ? pop() : -1;
-        load(c0, c1);
-        float qf[KP / 2];
-        line_operand<KP>(Qb, a.K, g.M, qi, h, qf);
+        int cur = __builtin_ctzll(any);
+        load(cur);
+        Parts qf[KP / 16];
+        line_parts<KP>(su, a.Q + (long)it.b * a.K * g.M, a.K, g.M, qi, h, qf);
+        const float alpha = a.alpha * kSplitUnscale;
         const int qc = min(qi, g.M - 1);
         const MRow mrow = mrow_of(a.mask ? a.mask + it.b * a.mask_bs : a.Q, a.mask ? g.M : 0, g.N, qc);
-        store(0, c0, c1);
+        store(0);
         __syncthreads();
         int buf = 0;
         while (true)
         {
-            const int n0 = pop(), n1 = CPS == 2 ? pop() : -1;
-            if (n0 >= 0) load(n0, n1);
-            const bool act0 = (lw.nz >> c0) & 1ull, act1 = c1 >= 0 && ((lw.nz >> c1) & 1ull);
-            if (act0 || act1)
+            const int nxt = rest ? __builtin_ctzll(rest) : -1;
+            const int jbase = 32 * (cell0 + cur);
+            const bool gen = (lw.gen >> cur) & 1ull, full = jbase + 32 <= g.N;
+            // The cell's mask before the next cell's tiles: loads are waited for in order, and the score
+            // chain covers these.
+            float mv[16];
+            if (gen) mask_row16(mrow, g.N, jbase, h, mv);
+            if (nxt >= 0) load(nxt);
+            if ((lw.nz >> cur) & 1ull)
             {
-                float x[CPS][16], cmax = kLowest;
-                // Every active cell's score chain first: the matrix core works
-                // on the second while the first one's scores are processed.
-                f32x16 scs[CPS];
-#pragma unroll
-                for (int t = 0; t < CPS; ++t)
-                    if (t ? act1 : act0) scs[t] = score_chain<KP, CPS == 2>(Ks[buf][t], qf, h, c);
-#pragma unroll
-                for (int t = 0; t < CPS; ++t)
+                float x[16];
+                const f32x16 sc = score_parts<KP>(L.k[buf], qf, h, c);
+                float cm;
+                if (full && !gen)
+                    cm = cell_scores<true, false>(sc, alpha, mrow, g.N, jbase, h, x);
+                else if (full)
+                    cm = cell_scores<true, true>(sc, alpha, mrow, g.N, jbase, h, x, mv);
+                else if (!gen)
+                    cm = cell_scores<false, false>(sc, alpha, mrow, g.N, jbase, h, x);
+                else
+                    cm = cell_scores<false, true>(sc, alpha, mrow, g.N, jbase, h, x, mv);
+                if constexpr (SST)
                 {
-                    const int cell = t ? c1 : c0;
-                    if (!(t ? act1 : act0))
-                    {
+                    // The cell's scores for the key-line pass, in this lane order.
+                    float* blk = a.S + (((long)it.b * g.RT + line) * g.CT + (cell0 + cur)) * 1024 + lane;
 #pragma unroll
-                        for (int r = 0; r < 16; ++r) x[t][r] = kNegInf;
-                        continue;
-                    }
-                    const int jbase = 32 * (cell0 + cell);
-                    const f32x16& sc = scs[t];
-                    const bool gen = (lw.gen >> cell) & 1ull, full = jbase + 32 <= g.N;
-                    float cm;
-                    if (full && !gen)
-                        cm = cell_scores<true, false>(sc, a.alpha, mrow, g.N, jbase, h, x[t]);
-                    else if (full)
-                        cm = cell_scores<true, true>(sc, a.alpha, mrow, g.N, jbase, h, x[t]);
-                    else if (!gen)
-                        cm = cell_scores<false, false>(sc, a.alpha, mrow, g.N, jbase, h, x[t]);
-                    else
-                        cm = cell_scores<false, true>(sc, a.alpha, mrow, g.N, jbase, h, x[t]);
-                    cmax = fmax_f(cmax, cm);
-                    if (a.S)
-                    {
-                        // The cell's scores for the key-line pass, in this lane order.
-                        float* blk = a.S + (((long)it.b * g.RT + line) * g.CT + (cell0 + cell)) * 1024 + lane;
-#pragma unroll
-                        for (int r = 0; r < 16; ++r) blk[r * 64] = x[t][r];
-                    }
+                    for (int r = 0; r < 16; ++r) blk[r * 64] = x[r];
                 }
-                cmax = fmax_f(cmax, __shfl_xor(cmax, 32));
-                const float mnew = fmax_f(mrun, cmax);
+                cm = fmax_f(cm, __shfl_xor(cm, 32));
+                const float mnew = fmax_f(mrun, cm);
                 if (__any(mnew != mrun))
                 {
                     const float scale = exp_neg(mrun - mnew);
@@ -626,31 +793,157 @@ __global__ __launch_bounds__(64 * kWaves, CPS == 1 ? 3 : 2) void k_flash_fwd(Fla
                     }
                     mrun = mnew;
                 }
-                // Rows still without an allowed key keep lowest() and only -inf scores.
-                const float mb = mrun == kLowest ? 0.0f : mrun * kLog2e;
+                if (__any(mrun == kLowest)) bad = not_finite(sc, bad);
+                // Rows still without an allowed key keep lowest() and only -inf scores. The weights are
+                // 2^24 exp(x - m): scaled for their split by the exponent's addend.
+                const float mb = (mrun == kLowest ? 0.0f : mrun * kLog2e) - 24.0f;
 #pragma unroll
-                for (int t = 0; t < CPS; ++t)
+                for (int r = 0; r < 16; ++r)
                 {
-                    if (!(t ? act1 : act0)) continue;
-#pragma unroll
-                    for (int r = 0; r < 16; ++r)
-                    {
-                        x[t][r] = __builtin_amdgcn_exp2f(__builtin_fmaf(x[t][r], kLog2e, -mb));
-                        lrun += x[t][r];
-                    }
-                    if constexpr (WITH_O) value_chain<DP, CPS == 2>(Vs[buf][t], x[t], h, c, o);
+                    x[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(x[r], kLog2e, -mb));
+                    lrun += x[r];
+                }
+                if constexpr (WITH_O)
+                {
+                    Parts w[2];
+                    weight_parts(su, x, w);
+                    value_parts<DP>(L.v[buf], w, h, c, o);
                 }
             }
-            if (n0 < 0) break;
-            store(buf ^ 1, n0, n1);
+            if (nxt < 0) break;
+            store(buf ^ 1);
             __syncthreads();
             buf ^= 1;
-            c0 = n0;
-            c1 = n1;
+            cur = nxt;
+            rest &= rest - 1;
+        }
+    }
+    lrun = (lrun + __shfl_xor(lrun, 32)) * (1.0f / kSplitScale);
+    bad = __builtin_fmaf(lrun, 0.0f, bad);
+    if constexpr (WITH_O)
+    {
+#pragma unroll
+        for (int u = 0; u < DU; ++u)
+        {
+            o[u] *= kSplitUnscale;
+            bad = not_finite(o[u], bad);
+        }
+    }
+    fwd_store<DP, WITH_O>(a, g, lw, it.b, line, it.rg, mrun, lrun, o);
+    return bad != 0.0f;
+}
+
+template <int KP, int DP, bool WITH_O, bool VDM>
+__device__ __forceinline__ void fwd_f32(const FlashFwdArgs& a, const FlashGeo& g, const Item& it, const LineWork& lw,
+                                     unsigned long long any, FwdLdsF32<KP, DP, WITH_O>& L)
+{
+    constexpr int DU = DP / 32;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, h = lane >> 5, c = lane & 31;
+    const int line = it.grp * kWaves + wave, qi = line * 32 + c;
+    float mrun = kLowest, lrun = 0.0f;
+    f32x16 o[DU];
+#pragma unroll
+    for (int u = 0; u < DU; ++u) o[u] = zero16();
+    if (any)
+    {
+        const int cell0 = it.rg * g.R;
+        const float* Qb = a.Q + (long)it.b * a.K * g.M;
+        const float* Kb = a.Kt + (long)it.b * a.K * g.N;
+        const float* Vb = WITH_O ? a.V + (long)it.b * g.N * a.D : nullptr;
+        TTile<KP> kt;
+        std::conditional_t<VDM, TTile<DP>, RTile<DP>> vt;   // V (D, N) or (N, D), staged [key][dim]
+        auto load = [&](int cell) {
+            kt.load(Kb, a.K, g.N, 32 * (cell0 + cell), threadIdx.x);
+            if constexpr (WITH_O && VDM) vt.load(Vb, a.D, g.N, 32 * (cell0 + cell), threadIdx.x);
+            if constexpr (WITH_O && !VDM) vt.load(Vb, a.D, a.D, g.N, 32 * (cell0 + cell), threadIdx.x);
+        };
+        auto store = [&](int buf) {
+            kt.store(L.k[buf], threadIdx.x);
+            if constexpr (WITH_O) vt.store(L.v[buf], threadIdx.x);
+        };
+        int cur = __builtin_ctzll(any);
+        unsigned long long rest = any & (any - 1);
+        load(cur);
+        float qf[KP / 2];
+        line_operand<KP>(Qb, a.K, g.M, qi, h, qf);
+        const int qc = min(qi, g.M - 1);
+        const MRow mrow = mrow_of(a.mask ? a.mask + it.b * a.mask_bs : a.Q, a.mask ? g.M : 0, g.N, qc);
+        store(0);
+        __syncthreads();
+        int buf = 0;
+        while (true)
+        {
+            const int nxt = rest ? __builtin_ctzll(rest) : -1;
+            if (nxt >= 0) load(nxt);
+            if ((lw.nz >> cur) & 1ull)
+            {
+                float x[16];
+                const f32x16 sc = score_chain<KP>(L.k[buf], qf, h, c);
+                const int jbase = 32 * (cell0 + cur);
+                const bool gen = (lw.gen >> cur) & 1ull;
+                float cm = gen ? cell_scores<false, true>(sc, a.alpha, mrow, g.N, jbase, h, x)
+                               : cell_scores<false, false>(sc, a.alpha, mrow, g.N, jbase, h, x);
+                if (a.S)
+                {
+                    float* blk = a.S + (((long)it.b * g.RT + line) * g.CT + (cell0 + cur)) * 1024 + lane;
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) blk[r * 64] = x[r];
+                }
+                cm = fmax_f(cm, __shfl_xor(cm, 32));
+                const float mnew = fmax_f(mrun, cm);
+                if (__any(mnew != mrun))
+                {
+                    const float scale = exp_neg(mrun - mnew);
+                    lrun *= scale;
+                    if constexpr (WITH_O)
+                    {
+#pragma unroll
+                        for (int u = 0; u < DU; ++u) o[u] *= scale;
+                    }
+                    mrun = mnew;
+                }
+                const float mb = mrun == kLowest ? 0.0f : mrun * kLog2e;
+#pragma unroll
+                for (int r = 0; r < 16; ++r)
+                {
+                    x[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(x[r], kLog2e, -mb));
+                    lrun += x[r];
+                }
+                if constexpr (WITH_O) value_chain<DP>(L.v[buf], x, h, c, o);
+            }
+            if (nxt < 0) break;
+            store(buf ^ 1);
+            __syncthreads();
+            buf ^= 1;
+            cur = nxt;
+            rest &= rest - 1;
         }
     }
     lrun += __shfl_xor(lrun, 32);
     fwd_store<DP, WITH_O>(a, g, lw, it.b, line, it.rg, mrun, lrun, o);
+}
+
+// SST: the rows' score blocks are stored (in straight code: a store behind a branch made the staging's wait for its
+// loads a wait for the stores as well).
+template <int KP, int DP, bool WITH_O, bool VDM, bool SST>
+__global__ __launch_bounds__(64 * kWaves, 2) void k_flash_fwd(FlashFwdSet t, FlashGeo g)
+{
+    union Lds
+    {
+        FwdLds<KP, DP, WITH_O> s;
+        FwdLdsF32<KP, DP, WITH_O> f;
+        __device__ Lds() {}
+    };
+    __shared__ __align__(16) Lds L;
+    __shared__ unsigned long long nz_s[kWaves];
+    const Item it = item_of(g);
+    const FlashFwdArgs a = row_args(t, g, it.b);
+    const LineWork lw = line_work(g, true, it.b, it.grp * kWaves + static_cast<int>(threadIdx.x >> 6), it.rg);
+    if ((threadIdx.x & 63) == 0) nz_s[threadIdx.x >> 6] = lw.nz;
+    __syncthreads();
+    const unsigned long long any = nz_s[0] | nz_s[1] | nz_s[2] | nz_s[3];
+    const bool bad = fwd_split<KP, DP, WITH_O, VDM, SST>(a, g, it, lw, any, L.s);
+    if (__syncthreads_or(bad)) fwd_f32<KP, DP, WITH_O, VDM>(a, g, it, lw, any, L.f);
 }
 
 // Merges of lines cut into several ranges (the k_flash_*_combine kernels):
@@ -1005,18 +1298,25 @@ __device__ __forceinline__ void cols_store(const FlashBwdArgs& a, const FlashGeo
         }
 }
 
+// The float32 chains (the split ones' fallback, see cols_split).
+template <int KP, bool GDO>
+struct ColsLdsF32
+{
+    float q[2][32][KP + 4];            // query tile [query][dim]
+    float o[2][32][KP + 4];            // dO tile [query][dim]
+    float g[GDO ? 1 : 2][32][KP + 4];  // G tile [query][dim] (GDO: the dO tile)
+};
 template <int KP, bool GDO, bool WDS, bool SST>
-__device__ __forceinline__ void cols_group(const FlashBwdArgs& a, const FlashGeo& g, int b, int grp, int rg,
-                                           float (*Qs)[32][KP + 4], float (*Os)[32][KP + 4],
-                                           float (*Gs)[32][KP + 4], float (*St)[3][32], unsigned long long* nz_s)
+__device__ __forceinline__ void cols_f32(const FlashBwdArgs& a, const FlashGeo& g, int b, int grp, int rg,
+                                         const LineWork& lw, unsigned long long any, ColsLdsF32<KP, GDO>& L,
+                                         float (*St)[3][32])
 {
     constexpr int DU = KP / 32;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, h = lane >> 5, c = lane & 31;
     const int line = grp * kWaves + wave, kj = line * 32 + c;
-    const LineWork lw = line_work(g, false, b, line, rg);
-    if (lane == 0) nz_s[wave] = lw.nz;
-    __syncthreads();
-    const unsigned long long any = nz_s[0] | nz_s[1] | nz_s[2] | nz_s[3];
+    auto& Qs = L.q;
+    auto& Os = L.o;
+    auto& Gs = L.g;
 
     f32x16 dk[DU], dv[DU];
 #pragma unroll
@@ -1131,7 +1431,7 @@ __device__ __forceinline__ void cols_group(const FlashBwdArgs& a, const FlashGeo
                     for (int r = 0; r < 16; ++r)
                     {
                         const int i = ibase + drow(r, h);
-                        if (i < g.M && kj < g.N) dsb[(long)i * g.N] = ds[r];
+                        if (i < g.M && kj < g.N) dsb[(long)i * g.N] = kSplitScale * ds[r];
                     }
                 }
             }
@@ -1154,17 +1454,229 @@ __device__ __forceinline__ void cols_group(const FlashBwdArgs& a, const FlashGeo
     cols_store<KP>(a, g, lw, b, line, rg, dk, dv);
 }
 
+// The key-line pass on the bf16 matrix cores: a cell of KP 64 is 72 MFMAs of 32
+// cycles (the dP, dV and dK chains; 24 more without the forward's score
+// blocks) where the float32 chains take 96 of 64. What bounds it: those 2304
+// cycles beside about 350 vector instructions (exp2, W and dS, the split of
+// both and of the staged tiles), two waves a SIMD. The dO tile is staged in
+// both forms (dP contracts over dims, dV over queries), G or Q in the value
+// form, Q in the score form only when the scores are formed here. W and dS
+// carry the split's scale 2^24 from the row factor 1 / l; dS is stored with
+// it. A workgroup whose results are not all finite runs again with cols_f32,
+// which KP 64 without score blocks runs at once: the split K line beside the
+// V line takes 60 registers more than two waves a SIMD have (the spills made
+// it slower than the float32 chains).
+template <int KP, bool GDO, bool SST>
+struct ColsLds
+{
+    static constexpr int NB = SST && GDO ? 2 : 1;   // buffers: two within 72 KB, two workgroups a CU
+    typename STile<KP>::Lds os[NB];                 // dO [query][dim]
+    typename VTile<KP>::Lds gv[NB];                 // dO or G [dim][query]
+    typename VTile<KP>::Lds qv[NB];                 // Q [dim][query]
+    bf16x8 qs[SST ? 1 : NB][3][SST ? 1 : 32 * KP / 8];   // Q [query][dim], without score blocks
+};
+template <int KP, bool GDO, bool WDS, bool SST>
+__device__ __forceinline__ bool cols_split(const FlashBwdArgs& a, const FlashGeo& g, int b, int grp, int rg,
+                                           const LineWork& lw, unsigned long long any, ColsLds<KP, GDO, SST>& L,
+                                           float (*St)[3][32])
+{
+    constexpr int DU = KP / 32, NB = ColsLds<KP, GDO, SST>::NB;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, h = lane >> 5, c = lane & 31;
+    const int line = grp * kWaves + wave, kj = line * 32 + c;
+    const SplitUnits su;
+    float bad = 0.0f;
+    f32x16 dk[DU], dv[DU];
+#pragma unroll
+    for (int u = 0; u < DU; ++u)
+    {
+        dk[u] = zero16();
+        dv[u] = zero16();
+    }
+    if (any)
+    {
+        const int cell0 = rg * g.R;
+        const float* Qb = a.Q + (long)b * a.K * g.M;
+        const float* Ob = a.dO + (long)b * a.Kd * g.M;
+        const float* Gb = a.G + (long)b * g.M * a.ldg;
+        const float* mb = a.m + (long)b * g.M;
+        const float* lb = a.l + (long)b * g.M;
+        const float* Rb = a.R + (long)b * g.M;
+        STile<KP> os, qs;
+        VTile<KP> gv, qv;
+        float st = 0.0f;
+        auto load = [&](int cell) {
+            const int i0 = 32 * (cell0 + cell);
+            os.load(Ob, a.Kd, g.M, i0);
+            if constexpr (GDO) gv.load(Ob, a.Kd, g.M, i0);
+            else gv.load_rows(Gb, a.ldg, a.K, g.M, i0);
+            qv.load(Qb, a.K, g.M, i0);
+            if constexpr (!SST) qs.load(Qb, a.K, g.M, i0);
+            if (threadIdx.x < 96)
+            {
+                const int i = i0 + static_cast<int>(threadIdx.x & 31), which = threadIdx.x >> 5;
+                float v = 0.0f;
+                if (i < g.M) v = which == 0 ? mb[i] : which == 1 ? lb[i] : Rb[i];
+                // m * log2(e) (0 for a row without allowed keys), 2^24 / l (0 for l = 0), R.
+                st = which == 0 ? (v == kLowest ? 0.0f : v * kLog2e)
+                                : which == 1 ? (v != 0.0f ? kSplitScale / v : 0.0f) : v;
+            }
+        };
+        auto store = [&](int buf) {
+            os.store(su, L.os[buf]);
+            if constexpr (GDO) gv.store(su, L.gv[buf]);
+            else gv.store_rows(su, L.gv[buf]);
+            qv.store(su, L.qv[buf]);
+            if constexpr (!SST) qs.store(su, L.qs[buf]);
+            if (threadIdx.x < 96) St[buf][threadIdx.x >> 5][threadIdx.x & 31] = st;
+        };
+        int cur = __builtin_ctzll(any);
+        unsigned long long rest = any & (any - 1);
+        load(cur);
+        Parts vf[KP / 16], kf[SST ? 1 : KP / 16];
+        line_parts<KP>(su, a.Vp + (long)b * a.Kd * g.N, a.Kd, g.N, kj, h, vf);
+        if constexpr (!SST) line_parts<KP>(su, a.Kt + (long)b * a.K * g.N, a.K, g.N, kj, h, kf);
+        // SST: this lane's key c in the forward's score blocks (r 64 + h 32 + q with drow(r, h) = c).
+        const float* sl = SST ? a.S + ((long)b * g.RT * g.CT + line) * 1024 + (4 * (c >> 3) + (c & 3)) * 64 +
+                                    ((c >> 2) & 1) * 32 + 4 * h
+                              : nullptr;
+        const int jc = min(kj, g.N - 1);
+        const float* mk = a.mask ? a.mask + b * a.mask_bs : nullptr;
+        FlashBwdArgs as = a;   // the scores' factor, for the scaled chain
+        as.alpha = a.alpha * kSplitUnscale;
+        const float alpha2 = a.alpha2 * kSplitUnscale;
+        const Rsrc dsb = rsrc(WDS ? a.dS + (long)b * g.M * g.N : a.Q, WDS ? (long)g.M * g.N : 0);
+        // SST: block (query tile cell0 + x, key tile line), queries drow(r, h), 4 at a time; issued before
+        // the dP chain, which covers it (a cell ahead it spills: 16 registers too many).
+        auto score_block = [&](int x, float* w) {
+            const float* blk = sl + (long)(cell0 + x) * g.CT * 1024;
+#pragma unroll
+            for (int g4 = 0; g4 < 4; ++g4)
+            {
+                const float4 v = *reinterpret_cast<const float4*>(blk + 8 * g4);
+                w[4 * g4 + 0] = v.x;
+                w[4 * g4 + 1] = v.y;
+                w[4 * g4 + 2] = v.z;
+                w[4 * g4 + 3] = v.w;
+            }
+        };
+        store(0);
+        __syncthreads();
+        int buf = 0;
+        while (true)
+        {
+            const int nxt = rest ? __builtin_ctzll(rest) : -1;
+            if (nxt >= 0) load(nxt);
+            if ((lw.nz >> cur) & 1ull)
+            {
+                const int ibase = 32 * (cell0 + cur);
+                float w[16];
+                const bool gen = (lw.gen >> cur) & 1ull, full = ibase + 32 <= g.M && (line + 1) * 32 <= g.N;
+                if constexpr (SST)
+                    score_block(cur, w);
+                else
+                {
+                    const f32x16 s = score_parts<KP>(L.qs[buf], kf, h, c);
+                    bad = not_finite(s, bad);
+                    if (full && !gen)
+                        col_scores<true, false>(s, as, mk, ibase, jc, kj, h, g.M, g.N, w);
+                    else if (full)
+                        col_scores<true, true>(s, as, mk, ibase, jc, kj, h, g.M, g.N, w);
+                    else if (!gen)
+                        col_scores<false, false>(s, as, mk, ibase, jc, kj, h, g.M, g.N, w);
+                    else
+                        col_scores<false, true>(s, as, mk, ibase, jc, kj, h, g.M, g.N, w);
+                }
+                const f32x16 p = score_parts<KP>(L.os[buf], vf, h, c);
+                if constexpr (SST)
+                    if (!full)
+                    {
+#pragma unroll
+                        for (int r = 0; r < 16; ++r)
+                            w[r] = (ibase + drow(r, h) < g.M && kj < g.N) ? w[r] : kNegInf;
+                    }
+                float ds[16];
+#pragma unroll
+                for (int r = 0; r < 16; ++r)
+                {
+                    const int ii = drow(r, h);
+                    w[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(w[r], kLog2e, -St[buf][0][ii])) * St[buf][1][ii];
+                    ds[r] = w[r] * (alpha2 * p[r] - St[buf][2][ii]);
+                }
+                if constexpr (WDS)
+                {
+                    // 2^24 dS of the cell, for the query-line pass (row i, key kj): one vector offset, the rows'
+                    // in scalar offsets, in a cell that lies inside the plane.
+                    const unsigned at = 4u * (static_cast<unsigned>(ibase + 4 * h) * g.N + kj);
+                    if (full)
+                    {
+#pragma unroll
+                        for (int r = 0; r < 16; ++r)
+                            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(ds[r]), dsb, at, 4 * drow(r, 0) * g.N,
+                                                                  0);
+                    }
+                    else
+                    {
+#pragma unroll
+                        for (int r = 0; r < 16; ++r)
+                            if (ibase + drow(r, h) < g.M && kj < g.N)
+                                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(ds[r]), dsb,
+                                                                      at + 4u * static_cast<unsigned>(drow(r, 0) * g.N),
+                                                                      0, 0);
+                    }
+                }
+                Parts wp[2];
+                // (the fences keep one chain's operands out of the other's registers)
+                __builtin_amdgcn_sched_barrier(0);
+                weight_parts(su, w, wp);
+                value_parts<KP>(L.gv[buf], wp, h, c, dv);
+                __builtin_amdgcn_sched_barrier(0);
+                weight_parts(su, ds, wp);
+                value_parts<KP>(L.qv[buf], wp, h, c, dk);
+            }
+            if (nxt < 0) break;
+            if constexpr (NB == 1) __syncthreads();
+            store(NB == 2 ? buf ^ 1 : 0);
+            __syncthreads();
+            if constexpr (NB == 2) buf ^= 1;
+            cur = nxt;
+            rest &= rest - 1;
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < DU; ++u)
+    {
+        dk[u] *= kSplitUnscale;
+        dv[u] *= kSplitUnscale;
+        bad = not_finite(dv[u], not_finite(dk[u], bad));
+    }
+    cols_store<KP>(a, g, lw, b, line, rg, dk, dv);
+    return bad != 0.0f;
+}
+
 template <int KP, bool GDO, bool WDS, bool SST = false>
 __global__ __launch_bounds__(64 * kWaves, 2) void k_flash_bwd_cols(FlashBwdSet t, FlashGeo g)
 {
-    __shared__ __align__(16) float Qs[2][32][KP + 4];   // query tile [query][dim]
-    __shared__ __align__(16) float Os[2][32][KP + 4];   // dO tile [query][dim]
-    __shared__ __align__(16) float Gs[GDO ? 1 : 2][32][KP + 4];   // G tile [query][dim] (GDO: the dO tile)
-    __shared__ float St[2][3][32];                      // m, 1/l, R of the tile's queries
+    union Lds
+    {
+        std::conditional_t<SST || KP == 32, ColsLds<KP, GDO, SST>, int> s;
+        ColsLdsF32<KP, GDO> f;
+        __device__ Lds() {}
+    };
+    __shared__ __align__(16) Lds L;
+    __shared__ float St[2][3][32];   // m, 1/l (times the scale), R of the tile's queries
     __shared__ unsigned long long nz_s[kWaves];
     const Item it = item_of(g);
     const FlashBwdArgs a = row_args(t, g, it.b);
-    cols_group<KP, GDO, WDS, SST>(a, g, it.b, it.grp, it.rg, Qs, Os, Gs, St, nz_s);
+    const LineWork lw = line_work(g, false, it.b, it.grp * kWaves + static_cast<int>(threadIdx.x >> 6), it.rg);
+    if ((threadIdx.x & 63) == 0) nz_s[threadIdx.x >> 6] = lw.nz;
+    __syncthreads();
+    const unsigned long long any = nz_s[0] | nz_s[1] | nz_s[2] | nz_s[3];
+    if constexpr (SST || KP == 32)
+    {
+        const bool bad = cols_split<KP, GDO, WDS, SST>(a, g, it.b, it.grp, it.rg, lw, any, L.s, St);
+        if (!__syncthreads_or(bad)) return;
+    }
+    cols_f32<KP, GDO, WDS, SST>(a, g, it.b, it.grp, it.rg, lw, any, L.f, St);
 }
 
 template <int KP>
@@ -1293,23 +1805,20 @@ __global__ __launch_bounds__(256) void k_flash_bwd_dq_combine(FlashBwdSet t, Fla
         }
 }
 
-// dQ from the stored dS: dQ_i = alpha sum_j dS_ij k_j over the non-empty cells
-// of the line's range, with the rows kernel's lines and ranges.
-template <int KP>
-__global__ __launch_bounds__(64 * kWaves, 3) void k_flash_bwd_dq(FlashBwdSet t, FlashGeo g)
+// dQ from the stored dS (2^24 dS): dQ_i = alpha sum_j dS_ij k_j over the
+// non-empty cells of the line's range, with the rows kernel's lines and
+// ranges. A cell is one chain, 24 bf16 MFMAs at KP 64 (split) or, in a
+// workgroup whose results are not all finite, 32 float32 ones.
+template <int KP, bool SPLIT>
+__device__ __forceinline__ bool dq_lines(const FlashBwdArgs& a, const FlashGeo& g, const Item& it, const LineWork& lw,
+                                         unsigned long long any, typename VTile<KP>::Lds* Ks,
+                                         float (*Kf)[32][KP + 4])
 {
     constexpr int DU = KP / 32;
-    __shared__ __align__(16) float Ks[2][32][KP + 4];   // key tile [key][dim]
-    __shared__ unsigned long long nz_s[kWaves];
-    const Item it = item_of(g);
-    const FlashBwdArgs a = row_args(t, g, it.b);
     const int b = it.b, rg = it.rg;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, h = lane >> 5, c = lane & 31;
     const int line = it.grp * kWaves + wave, qi = line * 32 + c;
-    const LineWork lw = line_work(g, true, b, line, rg);
-    if (lane == 0) nz_s[wave] = lw.nz;
-    __syncthreads();
-    const unsigned long long any = nz_s[0] | nz_s[1] | nz_s[2] | nz_s[3];
+    const SplitUnits su;
     f32x16 x[DU];
 #pragma unroll
     for (int u = 0; u < DU; ++u) x[u] = zero16();
@@ -1318,14 +1827,22 @@ __global__ __launch_bounds__(64 * kWaves, 3) void k_flash_bwd_dq(FlashBwdSet t, 
         const int cell0 = rg * g.R;
         const float* Kb = a.Kt + (long)b * a.K * g.N;
         const MRow dsrow = mrow_of(a.dS + (long)b * g.M * g.N, g.M, g.N, min(qi, g.M - 1));
-        TTile<KP> kt;
+        std::conditional_t<SPLIT, VTile<KP>, TTile<KP>> kt;
+        auto load = [&](int cell) {
+            if constexpr (SPLIT) kt.load(Kb, a.K, g.N, 32 * (cell0 + cell));
+            else kt.load(Kb, a.K, g.N, 32 * (cell0 + cell), threadIdx.x);
+        };
+        auto store = [&](int buf) {
+            if constexpr (SPLIT) kt.store(su, Ks[buf]);
+            else kt.store(Kf[buf], threadIdx.x);
+        };
         int cur = __builtin_ctzll(any);
         unsigned long long rest = any & (any - 1);
-        kt.load(Kb, a.K, g.N, 32 * (cell0 + cur), threadIdx.x);
+        load(cur);
         // This line's dS of a cell is loaded one cell ahead of its chain.
         float w[16];
         if ((lw.nz >> cur) & 1ull) mask_row16(dsrow, g.N, 32 * (cell0 + cur), h, w);
-        kt.store(Ks[0], threadIdx.x);
+        store(0);
         __syncthreads();
         int buf = 0;
         while (true)
@@ -1334,21 +1851,59 @@ __global__ __launch_bounds__(64 * kWaves, 3) void k_flash_bwd_dq(FlashBwdSet t, 
             float wn[16];
             if (nxt >= 0)
             {
-                kt.load(Kb, a.K, g.N, 32 * (cell0 + nxt), threadIdx.x);
+                load(nxt);
                 if ((lw.nz >> nxt) & 1ull) mask_row16(dsrow, g.N, 32 * (cell0 + nxt), h, wn);
             }
-            if ((lw.nz >> cur) & 1ull) value_chain<KP>(Ks[buf], w, h, c, x);
+            if ((lw.nz >> cur) & 1ull)
+            {
+                if constexpr (SPLIT)
+                {
+                    Parts wp[2];
+                    weight_parts(su, w, wp);
+                    value_parts<KP>(Ks[buf], wp, h, c, x);
+                }
+                else
+                    value_chain<KP>(Kf[buf], w, h, c, x);
+            }
             if (nxt < 0) break;
 #pragma unroll
             for (int r = 0; r < 16; ++r) w[r] = wn[r];
-            kt.store(Ks[buf ^ 1], threadIdx.x);
+            store(buf ^ 1);
             __syncthreads();
             buf ^= 1;
             cur = nxt;
             rest &= rest - 1;
         }
     }
+    float bad = 0.0f;
+#pragma unroll
+    for (int u = 0; u < DU; ++u)
+    {
+        x[u] *= SPLIT ? kSplitUnscale : 1.0f / kSplitScale;
+        if constexpr (SPLIT) bad = not_finite(x[u], bad);
+    }
     dq_store<KP>(a, g, lw, b, line, rg, x);
+    return bad != 0.0f;
+}
+template <int KP>
+__global__ __launch_bounds__(64 * kWaves, 3) void k_flash_bwd_dq(FlashBwdSet t, FlashGeo g)
+{
+    union Lds
+    {
+        typename VTile<KP>::Lds s[2];
+        float f[2][32][KP + 4];   // key tile [key][dim]
+        __device__ Lds() {}
+    };
+    __shared__ __align__(16) Lds L;
+    __shared__ unsigned long long nz_s[kWaves];
+    const Item it = item_of(g);
+    const FlashBwdArgs a = row_args(t, g, it.b);
+    const LineWork lw = line_work(g, true, it.b, it.grp * kWaves + static_cast<int>(threadIdx.x >> 6), it.rg);
+    if ((threadIdx.x & 63) == 0) nz_s[threadIdx.x >> 6] = lw.nz;
+    __syncthreads();
+    const unsigned long long any = nz_s[0] | nz_s[1] | nz_s[2] | nz_s[3];
+    const bool bad = dq_lines<KP, true>(a, g, it, lw, any, L.s, nullptr);
+    if (__syncthreads_or(bad)) dq_lines<KP, false>(a, g, it, lw, any, nullptr, L.f);
 }
 
 // Work order of a flash launch (one workgroup of 1024 threads). The weight of
@@ -1703,25 +2258,18 @@ int dq_pw(int KP) { return 32 * KP; }
 template <int KP, int DP, bool WITH_O>
 int launch_fwd(const FlashFwdSet& t, const FlashGeo& g0, size_t batch, const int* order, hipStream_t s)
 {
-    // Cells per step: one cell (3 workgroups per CU: 35 KB of LDS, <= 168
-    // VGPRs) when a line range holds >= 32 cells, two (2 per CU) for shorter
-    // ranges, where fewer barriers per cell pay more. Measured: causal
-    // (96 x 1024)^2 58 -> 71 TFLOP/s with one; causal (128 x 512)^2 and the
-    // document-masked rows 3-4 % faster with two.
     const dim3 grid(grid_of(g0, batch)), block(64 * kWaves);
-    const bool one = std::min(g0.R, g0.CT) >= 32;
     FlashGeo g = g0;
     g.order = order;
+    const bool sst = t.a[0].S != nullptr;   // (in every row of a launch or in none)
+    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, block, 0, s, t, g); };
     if (WITH_O && t.a[0].v_dm)
     {
-        if (one) hipLaunchKernelGGL((k_flash_fwd<KP, DP, WITH_O, true, 1>), grid, block, 0, s, t, g);
-        else hipLaunchKernelGGL((k_flash_fwd<KP, DP, WITH_O, true, 2>), grid, block, 0, s, t, g);
+        if (sst) go(k_flash_fwd<KP, DP, WITH_O, true, true>);
+        else go(k_flash_fwd<KP, DP, WITH_O, true, false>);
     }
-    else
-    {
-        if (one) hipLaunchKernelGGL((k_flash_fwd<KP, DP, WITH_O, false, 1>), grid, block, 0, s, t, g);
-        else hipLaunchKernelGGL((k_flash_fwd<KP, DP, WITH_O, false, 2>), grid, block, 0, s, t, g);
-    }
+    else if (sst) go(k_flash_fwd<KP, DP, WITH_O, false, true>);
+    else go(k_flash_fwd<KP, DP, WITH_O, false, false>);
     if (int rc = launch_status()) return rc;
     if (g.NR == 1) return 0;
     hipLaunchKernelGGL((k_flash_fwd_combine<DP, WITH_O>), dim3(static_cast<unsigned>(batch * g.RT)), dim3(256), 0, s,
@@ -1814,7 +2362,7 @@ int flash_build_rows_order(const unsigned char* const* cells, int rows, size_t h
     const FlashGeo gr = geo(batch, M, N, true, 0, cells[0], nullptr, per_batch_cls);
     const FlashGeo gc = geo(batch, M, N, false, 0, cells[0], nullptr, per_batch_cls);
     const FlashCls tab = cls_table(cells, rows, hpr, gr.cls_bs);
-    if (kind == 0) return build_order(gr, tab, batch, true, std::min(gr.R, gr.CT) >= 32 ? 3 : 2, at, s);
+    if (kind == 0) return build_order(gr, tab, batch, true, 2, at, s);
     if (kind == 1)
     {
         if (int rc = build_order(gr, tab, batch, true, 2, at, s)) return rc;

@@ -62,14 +62,14 @@ __device__ __forceinline__ bf16x2 split_part(const SplitUnits& u, float& x0, flo
     return p;
 }
 
-// The three parts of eight floats.
-__device__ __forceinline__ void split3(const SplitUnits& u, floatx8 x, bf16x8& h, bf16x8& m, bf16x8& l)
+// The three parts of eight floats that are scaled already.
+__device__ __forceinline__ void split3_scaled(const SplitUnits& u, floatx8 x, bf16x8& h, bf16x8& m, bf16x8& l)
 {
     uintx4 hv, mv, lv;
 #pragma unroll
     for (int p = 0; p < 4; ++p)
     {
-        float x0 = x[2 * p] * kSplitScale, x1 = x[2 * p + 1] * kSplitScale;
+        float x0 = x[2 * p], x1 = x[2 * p + 1];
         hv[p] = __builtin_bit_cast(unsigned, split_part(u, x0, x1));
         mv[p] = __builtin_bit_cast(unsigned, split_part(u, x0, x1));
         lv[p] = __builtin_bit_cast(unsigned, __builtin_convertvector((floatx2){x0, x1}, bf16x2));
@@ -77,6 +77,13 @@ __device__ __forceinline__ void split3(const SplitUnits& u, floatx8 x, bf16x8& h
     h = __builtin_bit_cast(bf16x8, hv);
     m = __builtin_bit_cast(bf16x8, mv);
     l = __builtin_bit_cast(bf16x8, lv);
+}
+// The three parts of eight floats.
+__device__ __forceinline__ void split3(const SplitUnits& u, floatx8 x, bf16x8& h, bf16x8& m, bf16x8& l)
+{
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x[e] *= kSplitScale;
+    split3_scaled(u, x, h, m, l);
 }
 
 // acc += the FM x FN blocks of 32 x 32 x 16 products' large parts, small += their five small ones; neighbouring

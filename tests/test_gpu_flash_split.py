@@ -1,0 +1,103 @@
+"""The attention chains formed from bf16 parts (csrc/split_bf16.hpp, k_flash.hip) at their edges.
+
+* Head dims and lengths around the tiles (32 tokens, 16-deep steps, dims padded to 32 or 64), forward
+  and backward with the forward's score blocks kept, also for lengths that are no whole tiles, against
+  float64. Bound: normwise 3e-6, about four times what float32 chains of this length show.
+* Inputs past the scaled range (2^104), keys excluded by -inf in K: the float32 chains.
+* Tiny gradients: no part is lost (the same bound).
+"""
+import numpy as np
+import pytest
+
+from helpers import causal_mask, normal
+
+pytestmark = pytest.mark.gpu
+TOL = 3e-6
+
+
+def chain(e, q, k, v, g, mask, H, T, d, alpha):
+    q, k, v, g, mk = (e.tensor(x) for x in (q, k, v, g, mask))
+    m = e.batched_matmul_reduce(q, k, H, "Max", True, False, alpha, True, mk)
+    l = e.batched_matmul_softmax_denom(q, k, m, H, True, False, alpha, mk)
+    vt = e.rearrange_3d(e.transpose(v), T, H, d)
+    o = e.batched_matmul_softmax_apply(q, k, vt, m, l, H, True, False, alpha, mk)
+    p = e.batched_matmul(g, v, H, True, False)
+    gt = e.rearrange_3d(e.transpose(g), T, H, d)
+    dq, r = e.batched_matmul_softmax_backward_q(q, k, p, m, l, H, True, False, alpha, mk)
+    dk, dv = e.batched_matmul_softmax_backward_kv(q, k, p, gt, r, m, l, H, True, False, alpha, mk)
+    del p, gt, vt
+    return [x.numpy() for x in (o, dq, dk, dv)]
+
+
+def exact(q, k, v, g, mask, H, T, d, alpha):
+    q, k, v, g = (x.astype(np.float64).reshape(H, d, T) for x in (q, k, v, g))
+    s = alpha * np.matmul(q.transpose(0, 2, 1), k) + mask.astype(np.float64)
+    p = np.exp(s - s.max(axis=2, keepdims=True))
+    p /= p.sum(axis=2, keepdims=True)
+    o = np.matmul(p, v.transpose(0, 2, 1))
+    dp = np.matmul(g.transpose(0, 2, 1), v)
+    ds = p * (dp - (p * dp).sum(axis=2, keepdims=True)) * alpha
+    dq = np.matmul(k, ds.transpose(0, 2, 1))
+    return [o.reshape(H * T, d), dq.reshape(H * d, T), np.matmul(q, ds).reshape(H * d, T),
+            np.matmul(g, p).reshape(H * d, T)]
+
+
+def rel(a, b):
+    return np.linalg.norm(a.astype(np.float64) - b) / np.linalg.norm(b)
+
+
+@pytest.mark.parametrize("H,T,d", [(3, 32, 64), (2, 33, 64), (5, 100, 64), (2, 129, 40), (3, 500, 64), (2, 257, 16),
+                                   (1, 64, 32), (4, 31, 20), (130, 70, 64), (2, 2050, 64)])
+@pytest.mark.parametrize("masked", [False, True])
+def test_edges(hip, H, T, d, masked):
+    rng = np.random.default_rng(H * 31 + T + d)
+    x = [normal(rng, (H * d, T)) for _ in range(4)]
+    mask = causal_mask(T)
+    if masked:   # general cells: finite values besides the excluded ones
+        mask = mask + normal(rng, (T, T))
+    got, ref = chain(hip, *x, mask, H, T, d, d ** -0.5), exact(*x, mask, H, T, d, d ** -0.5)
+    for n, a, b in zip(("o", "dq", "dk", "dv"), got, ref):
+        assert np.isfinite(a).all(), n
+        assert rel(a, b) <= TOL, (n, rel(a, b))
+
+
+@pytest.mark.parametrize("T,d", [(64, 64), (100, 32), (77, 64)])
+def test_values_past_the_scaled_range(hip, T, d):
+    """V of 1e33 (past 2^104) and Q of 1e32 against K of 1e-32, dO of 1e-30: the float32 chains."""
+    rng = np.random.default_rng(T)
+    H = 2
+    q, k = normal(rng, (H * d, T)) * np.float32(1e32), normal(rng, (H * d, T)) * np.float32(1e-32)
+    v, g = normal(rng, (H * d, T)) * np.float32(1e33), normal(rng, (H * d, T)) * np.float32(1e-30)
+    got, ref = chain(hip, q, k, v, g, causal_mask(T), H, T, d, 0.125), exact(q, k, v, g, causal_mask(T), H, T, d, 0.125)
+    for a, b in zip(got, ref):
+        assert np.isfinite(a).all()
+        assert rel(a, b) <= TOL
+
+
+@pytest.mark.parametrize("T", [64, 77])
+def test_minus_infinity_in_k(hip, T):
+    H, d = 2, 64
+    rng = np.random.default_rng(T)
+    q, k, v, g = (normal(rng, (H * d, T)) for _ in range(4))
+    q[5] = np.abs(q[5]) + 0.5
+    k[5, 3] = -np.inf          # head 0, key 3: every score of it is -inf
+    mask = causal_mask(T)
+    kk, mm = k.copy(), np.repeat(mask[None], H, 0).copy()
+    kk[5, 3] = 0.0
+    mm[0, :, 3] = -np.inf
+    mm[0, 3, 0] = 0.0          # (query 3 keeps other keys)
+    o = chain(hip, q, k, v, g, mask, H, T, d, 0.125)[0]
+    ref = exact(q, kk, v, g, mm, H, T, d, 0.125)[0]
+    assert rel(o, ref) <= TOL
+
+
+@pytest.mark.parametrize("scale", [1e-36, 1e-41])
+def test_tiny_gradients(hip, scale):
+    H, T, d = 3, 96, 64
+    rng = np.random.default_rng(7)
+    q, k, v = (normal(rng, (H * d, T)) for _ in range(3))
+    g = (normal(rng, (H * d, T)).astype(np.float64) * scale).astype(np.float32)
+    got, ref = chain(hip, q, k, v, g, causal_mask(T), H, T, d, 0.125), exact(q, k, v, g, causal_mask(T), H, T, d, 0.125)
+    quantum = 2.0 ** -149 * np.sqrt(got[3].size)
+    for a, b in zip(got[1:], ref[1:]):
+        assert np.linalg.norm(a.astype(np.float64) - b) <= TOL * np.linalg.norm(b) + T * quantum
