@@ -409,8 +409,9 @@ __device__ __forceinline__ void line_operand(const float* base, int dims, int T,
 //     score registers 8 s .. 8 s + 7 of step s, tokens 16 s + 4 h + 0..3 and
 //     + 8..11: the octet 2 s + h holds those tokens, so weights never move
 //     between lanes. Row u 32 + i holds dim DU i + u (the outputs' order).
-// Rows of 64 or 128 bytes, octets swapped so that 16 neighbouring rows' same
-// octet covers the LDS banks once. A cell of KP = DP = 64 is 48 MFMAs of 32
+// Rows of 64 or 128 bytes, octets swapped so that neither the 16-byte reads of
+// neighbouring rows' same octet (16 lanes at a time) nor the writes (8 lanes)
+// meet an LDS bank twice. A cell of KP = DP = 64 is 48 MFMAs of 32
 // cycles forward where the float32 chains take 64 of 64.
 typedef bf16x8 Parts[3];
 
@@ -422,7 +423,10 @@ struct STile
     floatx8 r;
     static __device__ __forceinline__ int slot(int tok, int o)
     {
-        return tok * OCT + (o ^ (OCT == 8 ? (tok >> 1) & 7 : (tok >> 2) & 3));
+        if constexpr (OCT == 8)
+            return tok * OCT + (o ^ ((tok >> 1 & 1) | ((tok >> 2 ^ tok >> 3) & 1) << 1 | ((tok ^ tok >> 3) & 1) << 2));
+        else
+            return tok * OCT + (o ^ ((tok >> 2) & 3) ^ (tok & 2));
     }
     static __device__ __forceinline__ bool mine() { return threadIdx.x < 32 * OCT; }
     // from a (dims, T) [dim][token] array: thread t holds token t % 32, dims 8 (t / 32) ..
@@ -448,7 +452,10 @@ struct VTile
 {
     typedef bf16x8 Lds[3][DP * 4];
     floatx8 r;
-    static __device__ __forceinline__ int slot(int row, int o) { return row * 4 + (o ^ ((row >> 2) & 3)); }
+    static __device__ __forceinline__ int slot(int row, int o)
+    {
+        return row * 4 + (o ^ ((row >> 2) & 3) ^ (row & 2));
+    }
     static __device__ __forceinline__ int row_of(int d) { return DP == 64 ? (d & 1) * 32 + (d >> 1) : d; }
     static __device__ __forceinline__ bool mine() { return threadIdx.x < 4 * DP; }
     // first token of octet o = 2 s + h: tokens 16 s + 4 h + 0..3 and + 8..11

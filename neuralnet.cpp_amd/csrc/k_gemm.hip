@@ -216,8 +216,12 @@ struct Operand
 };
 
 // LDS place of 8 k (slot s of 4) of a line: lines of 64 bytes, the slots
-// swapped so that 16 neighbouring lines' same slot covers the 64 banks once.
-__device__ __forceinline__ int lds_slot(int line, int s) { return line * 4 + (s ^ ((line >> 2) & 3)); }
+// swapped so that neither a 16-byte read of 32 neighbouring lines' same slot
+// (16 lanes at a time, lanes 0-3, 12-15, 20-23, 24-27 first) nor a write of 8
+// neighbouring lines' meets a bank twice (swapped by line / 4 alone, the
+// writes of operands stored along their lines did: 30 % of the LDS cycles of
+// the TN products).
+__device__ __forceinline__ int lds_slot(int line, int s) { return line * 4 + (s ^ ((line >> 2) & 3) ^ (line & 2)); }
 
 // Whole products and sums of KSEG segments (k runs through operand k / klen).
 struct SegNone
@@ -374,11 +378,23 @@ __global__ __launch_bounds__(64 * WM * WN, FM * FN == 4 ? 2 : 3) void k_gemm(
             int kt = 0;
             for (; kt + 2 < full; ++kt)
             {
-                // one block of straight code: the conversion and the LDS writes
-                // of stage kt + 1 issue in the shadow of stage kt's MFMAs
-                store((kt & 1) ^ 1);
-                load(kt + 2, false);
-                products(kt & 1);
+                // Waves w and w + 4 share a SIMD. The conversion of stage
+                // kt + 1 issues in the shadow of stage kt's MFMAs; with both
+                // operands k-contiguous the second four waves convert after
+                // them instead of before (NT 6144 x 768 x 8192 512 -> 500 us
+                // and 32000 x 768 x 2048 622 -> 601; NN and TN 0-4 % slower).
+                if (TB && wave >= WM * WN / 2)
+                {
+                    products(kt & 1);
+                    store((kt & 1) ^ 1);
+                    load(kt + 2, false);
+                }
+                else
+                {
+                    store((kt & 1) ^ 1);
+                    load(kt + 2, false);
+                    products(kt & 1);
+                }
                 __syncthreads();
             }
             for (; kt < nk; ++kt)
