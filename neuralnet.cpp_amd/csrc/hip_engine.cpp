@@ -3439,7 +3439,7 @@ Result<Tensor> HipEngine::elementwise_binary(BinaryOp op, const Tensor& A, const
     }
     // scores + mask of a deferred scores product (materialised attention): recorded.
     if (op == BinaryOp::Add && pgemm_ && same_t(A, pgemm_->C) && !has_buf(B, A.dev_ptr()) && A.size() &&
-        pgemm_->N == B.cols() && pgemm_->K <= 64)
+        pgemm_->N == B.cols() && pgemm_->K <= (pgemm_->M > 1 ? 128u : 64u))
     {
         NN_CHECK(settle_reads_({&B}));
         NN_CHECK(settle_madd_());

@@ -87,6 +87,10 @@ __device__ __forceinline__ float exp_neg(float x) { return __builtin_amdgcn_exp2
 // v_max_f32; for the finite and -inf scores here the same as (a < b ? b : a).
 __device__ __forceinline__ float fmax_f(float a, float b) { return __builtin_fmaxf(a, b); }
 
+// Waves a SIMD: two, or one for heads wider than 64, whose line operands and
+// accumulators take up to 400 registers and whose tiles 96 to 144 KB of LDS.
+constexpr int waves_per_simd(int KP, int DP = 32) { return KP == 128 || DP == 128 ? 1 : 2; }
+
 // Buffer loads with the hardware range check: a load whose byte offset is at
 // or past the resource's size returns 0 without touching memory, so padding
 // elements (offset kOob) are zero with no branch around the load. A resource
@@ -343,11 +347,23 @@ __device__ __forceinline__ void value_chain(const float (*tile)[DP + 4], const f
         float2 a[16];
 #pragma unroll
         for (int r = 0; r < 16; ++r) a[r] = *reinterpret_cast<const float2*>(&tile[drow(r, h)][2 * c]);
-    #pragma unroll
+#pragma unroll
         for (int r = 0; r < 16; ++r)
         {
             acc[0] = mfma(a[r].x, w[r], acc[0]);
             acc[1] = mfma(a[r].y, w[r], acc[1]);
+        }
+    }
+    else if constexpr (DU == 4)
+    {
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+        {
+            const float4 a = *reinterpret_cast<const float4*>(&tile[drow(r, h)][4 * c]);
+            acc[0] = mfma(a.x, w[r], acc[0]);
+            acc[1] = mfma(a.y, w[r], acc[1]);
+            acc[2] = mfma(a.z, w[r], acc[2]);
+            acc[3] = mfma(a.w, w[r], acc[3]);
         }
     }
     else
@@ -355,7 +371,7 @@ __device__ __forceinline__ void value_chain(const float (*tile)[DP + 4], const f
         float a[16];
 #pragma unroll
         for (int r = 0; r < 16; ++r) a[r] = tile[drow(r, h)][c];
-    #pragma unroll
+#pragma unroll
         for (int r = 0; r < 16; ++r) acc[0] = mfma(a[r], w[r], acc[0]);
     }
 }
@@ -368,22 +384,13 @@ __device__ __forceinline__ void value_chain2(const float (*tile)[DP + 4], const 
     constexpr int DU = DP / 32;
 #pragma unroll
     for (int r = 0; r < 16; ++r)
-    {
-        if constexpr (DU == 2)
+#pragma unroll
+        for (int u = 0; u < DU; ++u)
         {
-            const float2 a = *reinterpret_cast<const float2*>(&tile[drow(r, h)][2 * c]);
-            acc1[0] = mfma(a.x, w1[r], acc1[0]);
-            acc1[1] = mfma(a.y, w1[r], acc1[1]);
-            acc2[0] = mfma(a.x, w2[r], acc2[0]);
-            acc2[1] = mfma(a.y, w2[r], acc2[1]);
+            const float a = tile[drow(r, h)][DU * c + u];
+            acc1[u] = mfma(a, w1[r], acc1[u]);
+            acc2[u] = mfma(a, w2[r], acc2[u]);
         }
-        else
-        {
-            const float a = tile[drow(r, h)][c];
-            acc1[0] = mfma(a, w1[r], acc1[0]);
-            acc2[0] = mfma(a, w2[r], acc2[0]);
-        }
-    }
 }
 
 // Per-lane B operand of a score chain: reg[kk] = X(dim kk + KP/2*h, token t) of a (dims, T) array.
@@ -418,92 +425,118 @@ typedef bf16x8 Parts[3];
 template <int KP>
 struct STile
 {
-    static constexpr int OCT = KP / 8;
+    static constexpr int OCT = KP / 8, U = OCT > 8 ? OCT / 8 : 1;
     typedef bf16x8 Lds[3][32 * OCT];
-    floatx8 r;
+    floatx8 r[U];
     static __device__ __forceinline__ int slot(int tok, int o)
     {
-        if constexpr (OCT == 8)
-            return tok * OCT + (o ^ ((tok >> 1 & 1) | ((tok >> 2 ^ tok >> 3) & 1) << 1 | ((tok ^ tok >> 3) & 1) << 2));
-        else
-            return tok * OCT + (o ^ ((tok >> 2) & 3) ^ (tok & 2));
+        const int f = (tok >> 1 & 1) | ((tok >> 2 ^ tok >> 3) & 1) << 1 | ((tok ^ tok >> 3) & 1) << 2;
+        if constexpr (OCT == 16) return tok * OCT + (o ^ f ^ (tok & 8));
+        else if constexpr (OCT == 8) return tok * OCT + (o ^ f);
+        else return tok * OCT + (o ^ ((tok >> 2) & 3) ^ (tok & 2));
     }
     static __device__ __forceinline__ bool mine() { return threadIdx.x < 32 * OCT; }
-    // from a (dims, T) [dim][token] array: thread t holds token t % 32, dims 8 (t / 32) ..
+    // from a (dims, T) [dim][token] array: thread t holds token t % 32, octets t / 32 + 8 u of dims
     __device__ __forceinline__ void load(const float* base, int dims, int T, int t0)
     {
         if (!mine()) return;
         const Rsrc rs = rsrc(base, (long)dims * T);
         const int t = t0 + static_cast<int>(threadIdx.x & 31), d0 = 8 * static_cast<int>(threadIdx.x >> 5);
 #pragma unroll
-        for (int e = 0; e < 8; ++e)   // dims past the array fall past the resource by themselves
-            r[e] = bload(rs, oob_if_neg(4u * static_cast<unsigned>((d0 + e) * T + t), T - 1 - t));
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int e = 0; e < 8; ++e)   // dims past the array fall past the resource by themselves
+                r[u][e] = bload(rs, oob_if_neg(4u * static_cast<unsigned>((d0 + 64 * u + e) * T + t), T - 1 - t));
     }
     __device__ __forceinline__ void store(const SplitUnits& su, Lds& l) const
     {
         if (!mine()) return;
-        const int o = slot(threadIdx.x & 31, threadIdx.x >> 5);
-        split3(su, r, l[0][o], l[1][o], l[2][o]);
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+        {
+            const int o = slot(threadIdx.x & 31, (threadIdx.x >> 5) + 8 * u);
+            split3(su, r[u], l[0][o], l[1][o], l[2][o]);
+        }
     }
 };
 
 template <int DP>
 struct VTile
 {
+    static constexpr int U = DP > 64 ? DP / 64 : 1;
     typedef bf16x8 Lds[3][DP * 4];
-    floatx8 r;
+    floatx8 r[U];
     static __device__ __forceinline__ int slot(int row, int o)
     {
         return row * 4 + (o ^ ((row >> 2) & 3) ^ (row & 2));
     }
-    static __device__ __forceinline__ int row_of(int d) { return DP == 64 ? (d & 1) * 32 + (d >> 1) : d; }
+    static __device__ __forceinline__ int row_of(int d) { return d % (DP / 32) * 32 + d / (DP / 32); }
     static __device__ __forceinline__ bool mine() { return threadIdx.x < 4 * DP; }
     // first token of octet o = 2 s + h: tokens 16 s + 4 h + 0..3 and + 8..11
     static __device__ __forceinline__ int tok0(int o) { return 16 * (o >> 1) + 4 * (o & 1); }
-    // from a (dims, T) [dim][token] array: thread t holds dim t / 4, octet t % 4
+    // from a (dims, T) [dim][token] array: thread t holds dims t / 4 + 64 u, octet t % 4
     __device__ __forceinline__ void load(const float* base, int dims, int T, int t0)
     {
         if (!mine()) return;
         const Rsrc rs = rsrc(base, (long)dims * T);
-        const int d = threadIdx.x >> 2, t = t0 + tok0(threadIdx.x & 3);
-        if (t0 + 32 <= T)
-        {
-            const float4 x = bload4(rs, 4u * static_cast<unsigned>(d * T + t)),
-                         y = bload4(rs, 4u * static_cast<unsigned>(d * T + t + 8));
-            r = floatx8{x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};
-        }
-        else
+        const int t = t0 + tok0(threadIdx.x & 3);
 #pragma unroll
-            for (int e = 0; e < 8; ++e)
+        for (int u = 0; u < U; ++u)
+        {
+            const int d = static_cast<int>(threadIdx.x >> 2) + 64 * u;
+            if (t0 + 32 <= T)
             {
-                const int te = t + (e < 4 ? e : e + 4);
-                r[e] = bload(rs, oob_if_neg(4u * static_cast<unsigned>(d * T + te), T - 1 - te));
+                const float4 x = bload4(rs, 4u * static_cast<unsigned>(d * T + t)),
+                             y = bload4(rs, 4u * static_cast<unsigned>(d * T + t + 8));
+                r[u] = floatx8{x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};
             }
+            else
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+                {
+                    const int te = t + (e < 4 ? e : e + 4);
+                    r[u][e] = bload(rs, oob_if_neg(4u * static_cast<unsigned>(d * T + te), T - 1 - te));
+                }
+        }
     }
     __device__ __forceinline__ void store(const SplitUnits& su, Lds& l) const
     {
         if (!mine()) return;
-        const int o = slot(row_of(threadIdx.x >> 2), threadIdx.x & 3);
-        split3(su, r, l[0][o], l[1][o], l[2][o]);
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+        {
+            const int o = slot(row_of((threadIdx.x >> 2) + 64 * u), threadIdx.x & 3);
+            split3(su, r[u], l[0][o], l[1][o], l[2][o]);
+        }
     }
-    // from a (T, ld) [token][dim] array (dims < ncols): thread t holds dim t % DP, octet t / DP
+    // from a (T, ld) [token][dim] array (dims < ncols): thread t holds dim t % DP, octets t / DP + (256 / DP) u
     __device__ __forceinline__ void load_rows(const float* base, int ld, int ncols, int T, int t0)
     {
         if (!mine()) return;
         const Rsrc rs = rsrc(base, (long)T * ld);
-        const int d = threadIdx.x % DP, t = t0 + tok0(threadIdx.x / DP);
+        const int d = threadIdx.x % DP;
 #pragma unroll
-        for (int e = 0; e < 8; ++e)
+        for (int u = 0; u < U; ++u)
         {
-            const int te = t + (e < 4 ? e : e + 4);
-            r[e] = bload(rs, oob_if_neg(4u * static_cast<unsigned>(te * ld + d), (T - 1 - te) | (ncols - 1 - d)));
+            const int t = t0 + tok0(threadIdx.x / DP + 256 / DP * u);
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+            {
+                const int te = t + (e < 4 ? e : e + 4);
+                r[u][e] = bload(rs, oob_if_neg(4u * static_cast<unsigned>(te * ld + d),
+                                               (T - 1 - te) | (ncols - 1 - d)));
+            }
         }
     }
     __device__ __forceinline__ void store_rows(const SplitUnits& su, Lds& l) const
     {
         if (!mine()) return;
-        const int o = slot(row_of(threadIdx.x % DP), threadIdx.x / DP);
-        split3(su, r, l[0][o], l[1][o], l[2][o]);
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+        {
+            const int o = slot(row_of(threadIdx.x % DP), threadIdx.x / DP + 256 / DP * u);
+            split3(su, r[u], l[0][o], l[1][o], l[2][o]);
+        }
     }
 };
 
@@ -633,6 +666,9 @@ __device__ __forceinline__ void fwd_store(const FlashFwdArgs& a, const FlashGeo&
                 if (d0 >= a.D) continue;
                 if constexpr (DU == 2)
                     *reinterpret_cast<float2*>(orow + d0) = make_float2(o[0][r] * inv, o[1][r] * inv);
+                else if constexpr (DU == 4)
+                    *reinterpret_cast<float4*>(orow + d0) =
+                        make_float4(o[0][r] * inv, o[1][r] * inv, o[2][r] * inv, o[3][r] * inv);
                 else
                     orow[d0] = o[0][r] * inv;
             }
@@ -933,7 +969,7 @@ __device__ __forceinline__ void fwd_f32(const FlashFwdArgs& a, const FlashGeo& g
 // SST: the rows' score blocks are stored (in straight code: a store behind a branch made the staging's wait for its
 // loads a wait for the stores as well).
 template <int KP, int DP, bool WITH_O, bool VDM, bool SST>
-__global__ __launch_bounds__(64 * kWaves, 2) void k_flash_fwd(FlashFwdSet t, FlashGeo g)
+__global__ __launch_bounds__(64 * kWaves, waves_per_simd(KP, DP)) void k_flash_fwd(FlashFwdSet t, FlashGeo g)
 {
     union Lds
     {
@@ -1021,6 +1057,9 @@ __global__ __launch_bounds__(256) void k_flash_fwd_combine(FlashFwdSet t, FlashG
             }
             else if constexpr (DU == 2)
                 *reinterpret_cast<float2*>(a.O + row * a.D + d0) = make_float2(o[0][k] * inv, o[1][k] * inv);
+            else if constexpr (DU == 4)
+                *reinterpret_cast<float4*>(a.O + row * a.D + d0) =
+                    make_float4(o[0][k] * inv, o[1][k] * inv, o[2][k] * inv, o[3][k] * inv);
             else
                 a.O[row * a.D + d0] = o[0][k] * inv;
         }
@@ -1155,7 +1194,7 @@ __device__ __forceinline__ void rows_group(const FlashBwdArgs& a, const FlashGeo
 }
 
 template <int KP>
-__global__ __launch_bounds__(64 * kWaves, 2) void k_flash_bwd_rows(FlashBwdSet t, FlashGeo g)
+__global__ __launch_bounds__(64 * kWaves, waves_per_simd(KP)) void k_flash_bwd_rows(FlashBwdSet t, FlashGeo g)
 {
     __shared__ __align__(16) float Ks[2][32][KP + 4];   // key tile [key][dim]
     __shared__ __align__(16) float Vs[2][32][KP + 4];   // V' tile [key][dim]
@@ -1470,9 +1509,9 @@ __device__ __forceinline__ void cols_f32(const FlashBwdArgs& a, const FlashGeo& 
 // form, Q in the score form only when the scores are formed here. W and dS
 // carry the split's scale 2^24 from the row factor 1 / l; dS is stored with
 // it. A workgroup whose results are not all finite runs again with cols_f32,
-// which KP 64 without score blocks runs at once: the split K line beside the
-// V line takes 60 registers more than two waves a SIMD have (the spills made
-// it slower than the float32 chains).
+// which KP 64 and 128 without score blocks run at once: the split K line beside
+// the V line takes 60 registers more than there are (the spills made it
+// slower than the float32 chains).
 template <int KP, bool GDO, bool SST>
 struct ColsLds
 {
@@ -1661,7 +1700,7 @@ __device__ __forceinline__ bool cols_split(const FlashBwdArgs& a, const FlashGeo
 }
 
 template <int KP, bool GDO, bool WDS, bool SST = false>
-__global__ __launch_bounds__(64 * kWaves, 2) void k_flash_bwd_cols(FlashBwdSet t, FlashGeo g)
+__global__ __launch_bounds__(64 * kWaves, waves_per_simd(KP)) void k_flash_bwd_cols(FlashBwdSet t, FlashGeo g)
 {
     union Lds
     {
@@ -1893,7 +1932,7 @@ __device__ __forceinline__ bool dq_lines(const FlashBwdArgs& a, const FlashGeo& 
     return bad != 0.0f;
 }
 template <int KP>
-__global__ __launch_bounds__(64 * kWaves, 3) void k_flash_bwd_dq(FlashBwdSet t, FlashGeo g)
+__global__ __launch_bounds__(64 * kWaves, KP == 128 ? 2 : 3) void k_flash_bwd_dq(FlashBwdSet t, FlashGeo g)
 {
     union Lds
     {
@@ -2014,10 +2053,10 @@ __global__ __launch_bounds__(kOrderThreads) void k_flash_order(FlashGeo g, Flash
 
 // R_i = alpha2 sum_d dO(d, i) O(d, i): dO per batch (Kd, M) dim-major; O the
 // same, or (M, Kd) query-major when o_qm. A workgroup takes 64 rows (one per
-// lane); wave w sums dims [w q, (w+1) q), q = Kd / 4 <= 16, in two chains
+// lane); wave w sums dims [w q, (w+1) q), q = Kd / 4 <= KD / 4, in two chains
 // (even and odd dims), and wave 0 adds the four partials in wave order.
 // Query-major O rows are contiguous: the workgroup's 64 Kd floats are staged
-// through LDS. Loops run a fixed 16 steps over clamped addresses, so every
+// through LDS. Loops run KD / 4 steps over clamped addresses, so every
 // load is in flight at once. blockIdx.y: the row of a multi-row launch (its
 // own dO, O and R, `total` entries each).
 struct RowdotSet
@@ -2026,10 +2065,11 @@ struct RowdotSet
     const float* O[kFlashMaxRows];
     float* R[kFlashMaxRows];
 };
+template <int KD>
 __global__ __launch_bounds__(256) void k_flash_rowdot(RowdotSet set, int M, int Kd, long total, float alpha2, int o_qm)
 {
     __shared__ float part[4][64];
-    __shared__ float Ot[64][65];
+    __shared__ float Ot[64][KD + 1];
     const float* __restrict__ dO = set.dO[blockIdx.y];
     const float* __restrict__ O = set.O[blockIdx.y];
     float* __restrict__ R = set.R[blockIdx.y];
@@ -2041,11 +2081,11 @@ __global__ __launch_bounds__(256) void k_flash_rowdot(RowdotSet set, int M, int 
         // 64 rows x Kd floats, Kd / 4 per thread; past the last row reads 0.
         const long n = min(64L, total - t0) * Kd;
         const Rsrc rs = rsrc(O + t0 * Kd, n);
-        float v[16];
+        float v[KD / 4];
 #pragma unroll
-        for (int k = 0; k < 16; ++k) v[k] = bload(rs, 4u * static_cast<unsigned>(threadIdx.x + 256 * k));
+        for (int k = 0; k < KD / 4; ++k) v[k] = bload(rs, 4u * static_cast<unsigned>(threadIdx.x + 256 * k));
 #pragma unroll
-        for (int k = 0; k < 16; ++k)
+        for (int k = 0; k < KD / 4; ++k)
             if (k < q)
             {
                 const unsigned e = threadIdx.x + 256u * k;
@@ -2059,16 +2099,16 @@ __global__ __launch_bounds__(256) void k_flash_rowdot(RowdotSet set, int M, int 
         const long b = t / M, i = t % M;
         const float* p = dO + (b * Kd + d0) * M + i;
         const float* od = O + (b * Kd + d0) * M + i;
-        float pv[16], ov[16];
+        float pv[KD / 4], ov[KD / 4];
 #pragma unroll
-        for (int k = 0; k < 16; ++k)
+        for (int k = 0; k < KD / 4; ++k)
         {
             const int kc = min(k, q - 1);
             pv[k] = p[(long)kc * M];
             ov[k] = o_qm ? Ot[lane][d0 + kc] : od[(long)kc * M];
         }
 #pragma unroll
-        for (int k = 0; k < 16; ++k)
+        for (int k = 0; k < KD / 4; ++k)
             if (k < q) acc[k & 1] = __builtin_fmaf(pv[k], ov[k], acc[k & 1]);
     }
     part[wave][lane] = acc[0] + acc[1];
@@ -2102,7 +2142,9 @@ __global__ __launch_bounds__(256) void k_flash_classify(const float* __restrict_
 // ── host side ────────────────────────────────────────────────────────────────
 size_t align256(size_t x) { return (x + 255) / 256 * 256; }
 
-int pad32(size_t x) { return x <= 32 ? 32 : 64; }
+int pad32(size_t x) { return x <= 32 ? 32 : x <= 64 ? 64 : 128; }
+// The forward's padded value width: 128 when either width is above 64 (one kernel for those).
+int pad_value(size_t K, size_t D) { return K > 64 || D > 64 ? 128 : pad32(D); }
 
 // Ranges per line: R cells each, R a power of two in [8, 64] and at most 64
 // ranges per line. One range when there are enough workgroups to fill the GPU
@@ -2316,12 +2358,12 @@ int launch_bwd(const FlashBwdSet& t, const FlashGeo& gr0, const FlashGeo& gc0, s
 
 bool flash_supported(size_t batch, size_t M, size_t N, size_t K, size_t D)
 {
-    // Head dims up to 64 and value widths up to 64 in multiples of 4 (16-byte
+    // Head dims up to 128 and value widths up to 128 in multiples of 4 (16-byte
     // value rows); sizes that fit int; at most 2^30 cells over all batches.
     // Lines of at most 64 ranges of 64 cells: M, N <= 131072.
     // One batch entry's (M, N) mask or score gradients below 2 GiB (32-bit
     // buffer offsets).
-    return batch >= 1 && M >= 1 && N >= 1 && K >= 1 && K <= 64 && D >= 1 && D <= 64 && D % 4 == 0 &&
+    return batch >= 1 && M >= 1 && N >= 1 && K >= 1 && K <= 128 && D >= 1 && D <= 128 && D % 4 == 0 &&
            M <= (size_t{1} << 17) && N <= (size_t{1} << 17) && batch <= (size_t{1} << 20) &&
            M * N < (size_t{1} << 29) &&
            batch * ((M + 31) / 32) * ((N + 31) / 32) <= (size_t{1} << 30);
@@ -2340,7 +2382,7 @@ int flash_classify(const float* mask, size_t masks, long mask_bs, size_t M, size
 
 size_t flash_workspace_bytes(size_t batch, size_t M, size_t N, size_t K, size_t D, bool backward)
 {
-    if (!backward) return part_bytes(geo(batch, M, N, true, fwd_pw(pad32(D)), nullptr, nullptr), batch, true);
+    if (!backward) return part_bytes(geo(batch, M, N, true, fwd_pw(pad_value(K, D)), nullptr, nullptr), batch, true);
     const int KP = pad32(K);
     return std::max(part_bytes(geo(batch, M, N, true, rows_pw(KP), nullptr, nullptr), batch, true),
                     part_bytes(geo(batch, M, N, false, cols_pw(KP), nullptr, nullptr), batch, false));
@@ -2393,12 +2435,15 @@ int flash_forward_rows(const FlashFwdArgs* a, const unsigned char* const* cells,
     for (int r = 0; r < rows; ++r)
         if (!same_launch(a0, a[r]) || (a[r].mask && !cells[r])) return -1;
     const size_t batch = static_cast<size_t>(rows) * hpr;
-    const int KP = pad32(static_cast<size_t>(a0.K)), DP = a0.O ? pad32(static_cast<size_t>(a0.D)) : 32;
+    const int DP = a0.O ? pad_value(static_cast<size_t>(a0.K), static_cast<size_t>(a0.D)) : 32;
+    const int KP = DP == 128 ? 128 : pad32(static_cast<size_t>(a0.K));
     const FlashGeo g = geo(batch, static_cast<size_t>(a0.M), static_cast<size_t>(a0.N), true, fwd_pw(DP),
                            a0.mask ? cells[0] : nullptr, ws, a0.mask && a0.mask_bs != 0);
     if (g.NR > 1 && !ws) return -1;
     const FlashFwdSet t = fwd_set(a, cells, rows, hpr, g.cls_bs);
     const int* ow = a0.mask ? order : nullptr;
+    if (DP == 128) return launch_fwd<128, 128, true>(t, g, batch, ow, s);
+    if (KP == 128) return launch_fwd<128, 32, false>(t, g, batch, ow, s);
     if (!a0.O)
         return KP == 32 ? launch_fwd<32, 32, false>(t, g, batch, ow, s) : launch_fwd<64, 32, false>(t, g, batch, ow, s);
     if (KP == 32)
@@ -2428,6 +2473,7 @@ int flash_backward(const FlashBwdArgs& a, const unsigned char* cells, size_t bat
                                                          order_table_bytes(gr, batch))
                          : nullptr;
     const FlashBwdSet t = bwd_set(&a, &cl, 1, batch, gr.cls_bs);
+    if (KP == 128) return launch_bwd<128>(t, gr, gc, batch, orr, occ, s);
     return KP == 32 ? launch_bwd<32>(t, gr, gc, batch, orr, occ, s) : launch_bwd<64>(t, gr, gc, batch, orr, occ, s);
 }
 
@@ -2478,8 +2524,12 @@ int flash_backward_ds_rows(const FlashBwdArgs* a, const float* const* O, int o_q
     }
     const FlashBwdSet t = bwd_set(x, cells, rows, hpr, gr.cls_bs);
     const long total = static_cast<long>(hpr * M);
-    hipLaunchKernelGGL(k_flash_rowdot, dim3(static_cast<unsigned>((total + 63) / 64), static_cast<unsigned>(rows)),
-                       dim3(256), 0, s, rd, x[0].M, x[0].Kd, total, x[0].alpha2, o_qm ? 1 : 0);
+    auto rowdot = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>((total + 63) / 64), static_cast<unsigned>(rows)),
+                           dim3(256), 0, s, rd, x[0].M, x[0].Kd, total, x[0].alpha2, o_qm ? 1 : 0);
+    };
+    if (KP == 128) rowdot(k_flash_rowdot<128>);
+    else rowdot(k_flash_rowdot<64>);
     if (int rc = launch_status()) return rc;
     auto run = [&](auto kp) -> int {
         constexpr int P = decltype(kp)::value;
@@ -2506,6 +2556,7 @@ int flash_backward_ds_rows(const FlashBwdArgs* a, const float* const* O, int o_q
         }
         return 0;
     };
+    if (KP == 128) return run(std::integral_constant<int, 128>{});
     return KP == 32 ? run(std::integral_constant<int, 32>{}) : run(std::integral_constant<int, 64>{});
 }
 

@@ -10,6 +10,7 @@ import numpy as np
 import pytest
 
 from helpers import causal_mask, normal
+from test_gpu_attn_chain import attn_mask, check, inputs, run
 
 pytestmark = pytest.mark.gpu
 TOL = 3e-6
@@ -47,7 +48,8 @@ def rel(a, b):
 
 
 @pytest.mark.parametrize("H,T,d", [(3, 32, 64), (2, 33, 64), (5, 100, 64), (2, 129, 40), (3, 500, 64), (2, 257, 16),
-                                   (1, 64, 32), (4, 31, 20), (130, 70, 64), (2, 2050, 64)])
+                                   (1, 64, 32), (4, 31, 20), (130, 70, 64), (2, 2050, 64),
+                                   (2, 33, 68), (3, 100, 96), (2, 777, 128), (1, 32, 128), (5, 65, 124), (140, 40, 128)])
 @pytest.mark.parametrize("masked", [False, True])
 def test_edges(hip, H, T, d, masked):
     rng = np.random.default_rng(H * 31 + T + d)
@@ -61,7 +63,46 @@ def test_edges(hip, H, T, d, masked):
         assert rel(a, b) <= TOL, (n, rel(a, b))
 
 
-@pytest.mark.parametrize("T,d", [(64, 64), (100, 32), (77, 64)])
+@pytest.mark.parametrize("H,T,d", [(3, 100, 128), (2, 257, 96), (2, 70, 64), (2, 64, 32)])
+@pytest.mark.parametrize("how", ["no_blocks", "no_output"])
+def test_backward_without_the_forwards_work(hip, H, T, d, how):
+    """Without score blocks (no budget for them) the key-line pass forms the scores; without the forward's output
+    R comes from a pass over query lines."""
+    rng = np.random.default_rng(T + d)
+    x, mask, alpha = [normal(rng, (H * d, T)) for _ in range(4)], causal_mask(T), d ** -0.5
+    ref = exact(*x, mask, H, T, d, alpha)
+    if how == "no_blocks":
+        hip.set_score_budget(0)
+        try:
+            got = chain(hip, *x, mask, H, T, d, alpha)
+        finally:
+            hip.set_score_budget(8 << 30)
+    else:
+        q, k, v, g, mk = (hip.tensor(a) for a in (*x, mask))
+        m = hip.batched_matmul_reduce(q, k, H, "Max", True, False, alpha, True, mk)
+        l = hip.batched_matmul_softmax_denom(q, k, m, H, True, False, alpha, mk)
+        p = hip.batched_matmul(g, v, H, True, False)
+        gt = hip.rearrange_3d(hip.transpose(g), T, H, d)
+        dq, r = hip.batched_matmul_softmax_backward_q(q, k, p, m, l, H, True, False, alpha, mk)
+        dk, dv = hip.batched_matmul_softmax_backward_kv(q, k, p, gt, r, m, l, H, True, False, alpha, mk)
+        del p
+        got, ref = [a.numpy() for a in (dq, dk, dv)], ref[1:]
+    for a, b in zip(got, ref):
+        assert rel(a, b) <= TOL
+
+
+@pytest.mark.parametrize("B,H,T,dk", [(2, 2, 64, 128), (1, 3, 100, 96), (2, 1, 130, 72), (1, 2, 31, 128)])
+@pytest.mark.parametrize("kind", ["alibi", "doc_alibi"])
+def test_materialised_wide_heads(hip, cpu, B, H, T, dk, kind):
+    """The materialised path (scores + mask, softmax rows, products) with heads wider than 64, against the oracle."""
+    rng = np.random.default_rng(T + dk)
+    doc = [np.cumsum(rng.random(T) < 0.04) for _ in range(B)] if kind == "doc_alibi" else None
+    mask, arrs = attn_mask(B, H, T, doc_ids=doc), inputs(T, B * H, T, dk)
+    for kw in (dict(), dict(order="kq"), dict(read_A=True)):
+        check(run(hip, arrs, mask, B * H, T, dk ** -0.5, **kw), run(cpu, arrs, mask, B * H, T, dk ** -0.5, **kw))
+
+
+@pytest.mark.parametrize("T,d", [(64, 64), (100, 32), (77, 64), (77, 128)])
 def test_values_past_the_scaled_range(hip, T, d):
     """V of 1e33 (past 2^104) and Q of 1e32 against K of 1e-32, dO of 1e-30: the float32 chains."""
     rng = np.random.default_rng(T)
