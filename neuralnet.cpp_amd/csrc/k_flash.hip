@@ -837,9 +837,9 @@ __device__ __forceinline__ bool fwd_split(const FlashFwdArgs& a, const FlashGeo&
                     mrun = mnew;
                 }
                 if (__any(mrun == kLowest)) bad = not_finite(sc, bad);
-                // Rows still without an allowed key keep lowest() and only -inf scores. The weights are
-                // 2^24 exp(x - m): scaled for their split by the exponent's addend.
-                const float mb = (mrun == kLowest ? 0.0f : mrun * kLog2e) - 24.0f;
+                // Rows still without an allowed key keep lowest() and only -inf scores. (The split's scale
+                // is a product: an addend of 24 in the exponent costs it 4 bits.)
+                const float mb = mrun == kLowest ? 0.0f : mrun * kLog2e;
 #pragma unroll
                 for (int r = 0; r < 16; ++r)
                 {
@@ -848,6 +848,8 @@ __device__ __forceinline__ bool fwd_split(const FlashFwdArgs& a, const FlashGeo&
                 }
                 if constexpr (WITH_O)
                 {
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) x[r] *= kSplitScale;
                     Parts w[2];
                     weight_parts(su, x, w);
                     value_parts<DP>(L.v[buf], w, h, c, o);
@@ -861,7 +863,7 @@ __device__ __forceinline__ bool fwd_split(const FlashFwdArgs& a, const FlashGeo&
             rest &= rest - 1;
         }
     }
-    lrun = (lrun + __shfl_xor(lrun, 32)) * (1.0f / kSplitScale);
+    lrun += __shfl_xor(lrun, 32);
     bad = __builtin_fmaf(lrun, 0.0f, bad);
     if constexpr (WITH_O)
     {
