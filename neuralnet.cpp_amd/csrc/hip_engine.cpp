@@ -719,6 +719,9 @@ HipEngine::~HipEngine()
     for (void* e : stage_ev_)
         if (e) (void)hipEventDestroy(static_cast<hipEvent_t>(e));
     if (stage_) (void)hipHostFree(stage_);
+    for (void* e : read_ev_)
+        if (e) (void)hipEventDestroy(static_cast<hipEvent_t>(e));
+    if (read_stage_) (void)hipHostFree(read_stage_);
 }
 
 // ── GEMM event profile ──────────────────────────────────────────────────────
@@ -1885,14 +1888,72 @@ Result<Matrix> HipEngine::to_matrix(const Tensor& t)
     if (!t.is_gpu()) return fail("to_matrix: tensor is not GPU");
     NN_CHECK(settle_reads_({&t}));
     Matrix m(t.rows(), t.cols());
-    if (m.size())
-    {
-        auto s = static_cast<hipStream_t>(stream_);
-        if (hipMemcpyAsync(m.data(), D(t), m.size() * sizeof(float), hipMemcpyDeviceToHost, s) != hipSuccess)
-            return fail("to_matrix: device to host copy failed");
-    }
-    NN_CHECK(sync_());
+    NN_CHECK(read_into(t, m.data()));
     return m;
+}
+
+// The tensor into the caller's memory, by pinned slots: the copy to slot k + 1
+// runs while slot k is moved on. A copy to pageable memory goes through the
+// runtime's own staging and, before this, a Matrix in between: reading a
+// 50 M parameter model's gradients took 22 ms (9 GB/s), most of it the page
+// faults and moves of two fresh host copies.
+Result<void> HipEngine::read_into(const Tensor& t, Scalar* out)
+{
+    if (!t.is_gpu()) return fail("to_matrix: tensor is not GPU");
+    NN_CHECK(settle_reads_({&t}));
+    const std::size_t bytes = t.size() * sizeof(float);
+    auto s = static_cast<hipStream_t>(stream_);
+    if (bytes && !read_stage_)
+    {
+        for (void*& e : read_ev_)
+        {
+            hipEvent_t ev = nullptr;
+            if (!e && hipEventCreateWithFlags(&ev, hipEventDisableTiming) != hipSuccess)
+                return fail("HipEngine: hipEventCreate failed");
+            if (!e) e = ev;
+        }
+        if (hipHostMalloc(&read_stage_, 2 * kReadSlot, hipHostMallocDefault) != hipSuccess)
+        {
+            (void)hipGetLastError();
+            read_stage_ = nullptr;
+        }
+    }
+    if (bytes && !read_stage_)   // no pinned memory to be had: straight to the caller's
+    {
+        if (hipMemcpyAsync(out, D(t), bytes, hipMemcpyDeviceToHost, s) != hipSuccess)
+            return fail("to_matrix: device to host copy failed");
+        return sync_();
+    }
+    if (bytes <= kReadSlot)
+    {
+        if (bytes && hipMemcpyAsync(read_stage_, D(t), bytes, hipMemcpyDeviceToHost, s) != hipSuccess)
+            return fail("to_matrix: device to host copy failed");
+        NN_CHECK(sync_());
+        if (bytes) std::memcpy(out, read_stage_, bytes);
+        return {};
+    }
+    const char* src = reinterpret_cast<const char*>(D(t));
+    char* dst = reinterpret_cast<char*>(out);
+    auto slot = [&](std::size_t k) { return static_cast<char*>(read_stage_) + (k & 1) * kReadSlot; };
+    const std::size_t chunks = (bytes + kReadSlot - 1) / kReadSlot;
+    for (std::size_t k = 0; k <= chunks; ++k)
+    {
+        if (k < chunks)
+        {
+            const std::size_t n = std::min(kReadSlot, bytes - k * kReadSlot);
+            if (hipMemcpyAsync(slot(k), src + k * kReadSlot, n, hipMemcpyDeviceToHost, s) != hipSuccess ||
+                hipEventRecord(static_cast<hipEvent_t>(read_ev_[k & 1]), s) != hipSuccess)
+                return fail("to_matrix: device to host copy failed");
+        }
+        if (k > 0)
+        {
+            if (hipEventSynchronize(static_cast<hipEvent_t>(read_ev_[(k - 1) & 1])) != hipSuccess)
+                return fail("to_matrix: device to host copy failed");
+            const std::size_t at = (k - 1) * kReadSlot;
+            std::memcpy(dst + at, slot(k - 1), std::min(kReadSlot, bytes - at));
+        }
+    }
+    return sync_();
 }
 
 Result<void> HipEngine::copy_from(Tensor& dst, const Matrix& src)

@@ -14,6 +14,7 @@
 //     -inf excludes a position, a finite value is added to the score.
 #pragma once
 
+#include <algorithm>
 #include <cstddef>
 #include <cstdint>
 #include <span>
@@ -50,6 +51,13 @@ public:
     [[nodiscard]] virtual Tensor create_tensor(std::size_t rows, std::size_t cols) = 0;
     [[nodiscard]] virtual Result<Tensor> from_matrix(const Matrix& m) = 0;
     [[nodiscard]] virtual Result<Matrix> to_matrix(const Tensor& t) = 0;
+    // to_matrix into the caller's t.size() floats (no reference counterpart: its hosts take the Matrix).
+    [[nodiscard]] virtual Result<void> read_into(const Tensor& t, Scalar* out)
+    {
+        NN_TRY(m, to_matrix(t));
+        std::copy(m.data(), m.data() + m.size(), out);
+        return {};
+    }
     [[nodiscard]] virtual Result<void> copy_from(Tensor& dst, const Matrix& src) = 0;
     [[nodiscard]] virtual Result<Tensor> clone(const Tensor& src) = 0;
 

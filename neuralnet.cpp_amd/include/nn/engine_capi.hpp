@@ -61,10 +61,8 @@ inline void* tensor_from_host(EngineHandle* e, const float* data, std::size_t r,
 
 inline int tensor_to_host(EngineHandle* e, const void* h, float* out)
 {
-    auto m = e->eng->to_matrix(*T(h));
-    if (!m) return set_error(m.error().message);
-    if (m->size()) std::memcpy(out, m->data(), m->size() * sizeof(float));
-    return 0;
+    auto r = e->eng->read_into(*T(h), out);
+    return r ? 0 : set_error(r.error().message);
 }
 
 inline int tensor_copy_from_host(EngineHandle* e, void* h, const float* data)
@@ -332,10 +330,8 @@ inline int gpt_set_param(GptSession* g, std::size_t i, const float* data)
 
 inline int gpt_read(GptSession* g, const Tensor& t, float* out)
 {
-    auto m = g->eng->to_matrix(t);
-    if (!m) return set_error(m.error().message);
-    std::memcpy(out, m->data(), m->size() * sizeof(float));
-    return 0;
+    auto r = g->eng->read_into(t, out);
+    return r ? 0 : set_error(r.error().message);
 }
 
 inline int gpt_set_doc_ids(GptSession* g, const std::uint64_t* ids, std::size_t n)

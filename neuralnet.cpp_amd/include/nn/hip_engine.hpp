@@ -73,6 +73,7 @@ public:
     Tensor create_tensor(std::size_t rows, std::size_t cols) override;
     Result<Tensor> from_matrix(const Matrix& m) override;
     Result<Matrix> to_matrix(const Tensor& t) override;
+    Result<void> read_into(const Tensor& t, Scalar* out) override;
     Result<void> copy_from(Tensor& dst, const Matrix& src) override;
     Result<Tensor> clone(const Tensor& src) override;
 
@@ -377,6 +378,11 @@ private:
     void* stage_ = nullptr;
     std::vector<void*> stage_ev_;
     std::size_t stage_next_ = 0;
+    // Two pinned slots for reads (read_into): while one is copied out to the
+    // caller's memory the other is being filled.
+    static constexpr std::size_t kReadSlot = std::size_t(2) << 20;
+    void* read_stage_ = nullptr;
+    void* read_ev_[2] = {nullptr, nullptr};
 
     bool ok_ = false;
     std::string init_error_;
