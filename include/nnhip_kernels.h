@@ -27,7 +27,7 @@ extern "C" {
 #pragma GCC visibility push(default) /* the library is built with hidden visibility */
 #endif
 
-/* ── GEMM (fp32 MFMA) ────────────────────────────────────────────────────
+/* ── GEMM (float32, formed from bf16 parts on the matrix cores) ────────────────────────────────────────────────────
  * C (M,N) = alpha * op(A) op(B); A stored (A_rows, A_cols), B stored (B_rows, B_cols).
  * Replaces cuda_matmul / cuda_matmul_with_handle (cuda_kernels.h:24-43). */
 int nnhip_matmul(const float* A, const float* B, float* C, size_t A_rows, size_t A_cols, size_t B_rows,
@@ -184,8 +184,8 @@ int nnhip_gemv_group_rmsnorm(const float* const* R, const float* x, const nnhip_
  * the library, one per GPU, NNHIP_GEMM_NOALLOC_SCRATCH_BYTES (64 MiB) in size and held until the process
  * ends. Same plan, kernels and summation order as nnhip_gemm given nnhip_gemm_workspace_bytes(M, N, K,
  * batch) bytes of workspace, so the results are identical. Returns -6, launching nothing, when that
- * workspace size exceeds NNHIP_GEMM_NOALLOC_SCRATCH_BYTES: products whose output grid fills the GPU need
- * none; among the config-4 step's, the long-K ones into small outputs (768 x 8192 from K = 6144 or
+ * workspace size exceeds NNHIP_GEMM_NOALLOC_SCRATCH_BYTES: products with K below 1024 need none; among
+ * the config-4 step's, the long-K ones into small outputs (768 x 8192 from K = 6144 or
  * 32000, the 6144 x 768 and 768 x 3072 weight gradients) need 72-144 MiB and are rejected. All calls on
  * one GPU share its scratch: calls that may overlap in time on one GPU (other streams, other threads) race
  * and must be ordered by the caller. */
@@ -315,7 +315,7 @@ int nnhip_bmm_softmax_backward_kv(const float* A, const float* B, const float* P
  * Q per batch (K,M) (the transA = 1 operand), K per batch (K,N) (transB = 0), V per batch (N,D),
  * dO per batch (Kd,M) and V' per batch (Kd,N) (P_ij = alpha2 sum_k dO(k,i) V'(k,j), recomputed, never
  * stored), G per batch (M,ldg). Supported when nnhip_flash_supported(batch, M, N, max(K,Kd), D)
- * (K, Kd <= 64; D <= 64, D % 4 == 0); the backward also needs K % 4 == 0, ldg % 4 == 0. Fully masked
+ * (K, Kd <= 128; D <= 128, D % 4 == 0); the backward also needs K % 4 == 0, ldg % 4 == 0. Fully masked
  * 32x32 cells are skipped; long rows are split over workgroups and combined in a fixed order. */
 int nnhip_flash_supported(size_t batch, size_t M, size_t N, size_t K, size_t D);
 /* Mask cell table: one byte per 32x32 cell of the (M,N) mask (0 all -inf, 1 all zero, 2 general), the
