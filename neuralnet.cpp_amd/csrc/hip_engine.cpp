@@ -1903,6 +1903,7 @@ Result<void> HipEngine::read_into(const Tensor& t, Scalar* out)
     NN_CHECK(settle_reads_({&t}));
     const std::size_t bytes = t.size() * sizeof(float);
     auto s = static_cast<hipStream_t>(stream_);
+    std::lock_guard<std::mutex> lk(read_mu_);
     if (bytes && !read_stage_)
     {
         for (void*& e : read_ev_)

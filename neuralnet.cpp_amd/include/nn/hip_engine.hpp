@@ -37,6 +37,7 @@
 #pragma once
 
 #include <memory>
+#include <mutex>
 #include <optional>
 #include <string>
 #include <unordered_set>
@@ -381,6 +382,7 @@ private:
     // Two pinned slots for reads (read_into): while one is copied out to the
     // caller's memory the other is being filled.
     static constexpr std::size_t kReadSlot = std::size_t(2) << 20;
+    std::mutex read_mu_;   // the slots serve one read at a time, also from several threads
     void* read_stage_ = nullptr;
     void* read_ev_[2] = {nullptr, nullptr};
 
