@@ -14,7 +14,8 @@ part: the fused causal-attention primitives on BASELINE config 2 (forward:
 bmm_reduce Max -> softmax_denom -> softmax_apply) and config 5 (document-masked
 forward + backward over the 8 packed rows), as algorithmic TFLOP/s (4*d*P
 forward, 8*d*P backward over the P allowed (query, key) pairs) and as a
-fraction of the fp32 MFMA peak, timed with HIP events on the engine's stream
+fraction of the fp32 MFMA peak (the metric's own yardstick: the kernels run on the
+bf16 cores, whose sixth is 417), timed with HIP events on the engine's stream
 at a steady clock (0.25 s of untimed calls first, then at least 20 ms timed).
 `cpu_baseline` runs the CPU restatement of the reference CpuEngine (oracle/,
 loaded only for this leg) on a bounded sample of the same workload: the
@@ -549,8 +550,8 @@ def _oracle(threads):
 
 
 def _cpu_threads():
-    """hardware_concurrency is the reference's pool size (core_threadpool.hpp:612); a GPU box lends one
-    GPU's job 16 of its host's CPUs, so the pool is capped at 16 (NNORACLE_THREADS overrides)."""
+    """hardware_concurrency is the reference's pool size (core_threadpool.hpp:612); a shared host lends one
+    GPU's job 16 of its CPUs, so the pool is capped at 16 (NNORACLE_THREADS overrides)."""
     return int(os.environ.get("NNORACLE_THREADS", "0")) or min(len(os.sched_getaffinity(0)), 16)
 
 

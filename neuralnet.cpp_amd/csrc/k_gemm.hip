@@ -19,9 +19,9 @@
 // vector instructions an element staged (1/128 + 1/256 elements a product in
 // the 256 x 128 tile). K advances 32 at a time. 256 x 128 tiles (8 waves, one
 // workgroup a CU) have two LDS buffers and convert stage k + 1 in the shadow
-// of stage k's MFMAs, with stage k + 2's loads in flight; the 4-wave tiles
-// have one buffer, so that two or three workgroups share a CU and cover each
-// other's conversions. Measured on MI355X, float32 MFMA before -> now:
+// of stage k's MFMAs, with stage k + 2's loads in flight; 128 x 64 tiles (4
+// waves) have one, so that two or three workgroups share a CU and cover each
+// other's conversions; 64 x 64 tiles (4 waves) have two. Measured on MI355X, float32 MFMA before -> now:
 // 6144 x 8192 x 768 126 -> 186 TFLOP/s, 4096^3 126 -> 204. The same loop
 // without the conversions runs 210 and 237; the bf16 cores alone would give
 // 348. Tile ids are remapped so that each XCD (own L2) works on a contiguous,
