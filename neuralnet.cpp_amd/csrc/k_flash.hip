@@ -1479,7 +1479,7 @@ __device__ __forceinline__ void cols_f32(const FlashBwdArgs& a, const FlashGeo& 
                     for (int r = 0; r < 16; ++r)
                     {
                         const int i = ibase + drow(r, h);
-                        if (i < g.M && kj < g.N) dsb[(long)i * g.N] = kSplitScale * ds[r];
+                        if (i < g.M && kj < g.N) dsb[(long)i * g.N] = ds[r];
                     }
                 }
             }
@@ -1509,8 +1509,9 @@ __device__ __forceinline__ void cols_f32(const FlashBwdArgs& a, const FlashGeo& 
 // both and of the staged tiles), two waves a SIMD. The dO tile is staged in
 // both forms (dP contracts over dims, dV over queries), G or Q in the value
 // form, Q in the score form only when the scores are formed here. W and dS
-// carry the split's scale 2^24 from the row factor 1 / l; dS is stored with
-// it. A workgroup whose results are not all finite runs again with cols_f32,
+// carry the split's scale 2^24 from the row factor 1 / l; dS is stored without
+// it (a stored 2^24 dS would be infinite from dS = 2^104 on, for the float32
+// chain of the dQ pass as well). A workgroup whose results are not all finite runs again with cols_f32,
 // which KP 64 and 128 without score blocks run at once: the split K line beside
 // the V line takes 60 registers more than there are (the spills made it
 // slower than the float32 chains).
@@ -1652,22 +1653,22 @@ __device__ __forceinline__ bool cols_split(const FlashBwdArgs& a, const FlashGeo
                 }
                 if constexpr (WDS)
                 {
-                    // 2^24 dS of the cell, for the query-line pass (row i, key kj): one vector offset, the rows'
-                    // in scalar offsets, in a cell that lies inside the plane.
+                    // dS of the cell, for the query-line pass (row i, key kj): one vector offset, the rows' in
+                    // scalar offsets, in a cell that lies inside the plane.
                     const unsigned at = 4u * (static_cast<unsigned>(ibase + 4 * h) * g.N + kj);
                     if (full)
                     {
 #pragma unroll
                         for (int r = 0; r < 16; ++r)
-                            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(ds[r]), dsb, at, 4 * drow(r, 0) * g.N,
-                                                                  0);
+                            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(ds[r] * (1.0f / kSplitScale)), dsb, at,
+                                                                  4 * drow(r, 0) * g.N, 0);
                     }
                     else
                     {
 #pragma unroll
                         for (int r = 0; r < 16; ++r)
                             if (ibase + drow(r, h) < g.M && kj < g.N)
-                                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(ds[r]), dsb,
+                                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(ds[r] * (1.0f / kSplitScale)), dsb,
                                                                       at + 4u * static_cast<unsigned>(drow(r, 0) * g.N),
                                                                       0, 0);
                     }
@@ -1853,7 +1854,7 @@ __global__ __launch_bounds__(256) void k_flash_bwd_dq_combine(FlashBwdSet t, Fla
         }
 }
 
-// dQ from the stored dS (2^24 dS): dQ_i = alpha sum_j dS_ij k_j over the
+// dQ from the stored dS: dQ_i = alpha sum_j dS_ij k_j over the
 // non-empty cells of the line's range, with the rows kernel's lines and
 // ranges. A cell is one chain, 24 bf16 MFMAs at KP 64 (split) or, in a
 // workgroup whose results are not all finite, 32 float32 ones.
@@ -1907,6 +1908,8 @@ __device__ __forceinline__ bool dq_lines(const FlashBwdArgs& a, const FlashGeo& 
                 if constexpr (SPLIT)
                 {
                     Parts wp[2];
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) w[r] *= kSplitScale;
                     weight_parts(su, w, wp);
                     value_parts<KP>(Ks[buf], wp, h, c, x);
                 }
@@ -1927,8 +1930,9 @@ __device__ __forceinline__ bool dq_lines(const FlashBwdArgs& a, const FlashGeo& 
 #pragma unroll
     for (int u = 0; u < DU; ++u)
     {
-        x[u] *= SPLIT ? kSplitUnscale : 1.0f / kSplitScale;
-        if constexpr (SPLIT) bad = not_finite(x[u], bad);
+        if constexpr (!SPLIT) continue;
+        x[u] *= kSplitUnscale;
+        bad = not_finite(x[u], bad);
     }
     dq_store<KP>(a, g, lw, b, line, rg, x);
     return bad != 0.0f;

@@ -4,11 +4,12 @@
   and backward with the forward's score blocks kept, also for lengths that are no whole tiles, against
   float64. Bound: normwise 3e-6, about four times what float32 chains of this length show.
 * Inputs past the scaled range (2^104), keys excluded by -inf in K: the float32 chains.
-* Tiny gradients: no part is lost (the same bound).
+* Tiny gradients: no part is lost (the same bound). Score gradients past 2^104: float32 as well.
 """
 import numpy as np
 import pytest
 
+import nnengine
 from helpers import causal_mask, normal
 from test_gpu_attn_chain import attn_mask, check, inputs, run
 
@@ -16,13 +17,13 @@ pytestmark = pytest.mark.gpu
 TOL = 3e-6
 
 
-def chain(e, q, k, v, g, mask, H, T, d, alpha):
+def chain(e, q, k, v, g, mask, H, T, d, alpha, alpha2=1.0):
     q, k, v, g, mk = (e.tensor(x) for x in (q, k, v, g, mask))
     m = e.batched_matmul_reduce(q, k, H, "Max", True, False, alpha, True, mk)
     l = e.batched_matmul_softmax_denom(q, k, m, H, True, False, alpha, mk)
     vt = e.rearrange_3d(e.transpose(v), T, H, d)
     o = e.batched_matmul_softmax_apply(q, k, vt, m, l, H, True, False, alpha, mk)
-    p = e.batched_matmul(g, v, H, True, False)
+    p = e.batched_matmul(g, v, H, True, False, alpha2)
     gt = e.rearrange_3d(e.transpose(g), T, H, d)
     dq, r = e.batched_matmul_softmax_backward_q(q, k, p, m, l, H, True, False, alpha, mk)
     dk, dv = e.batched_matmul_softmax_backward_kv(q, k, p, gt, r, m, l, H, True, False, alpha, mk)
@@ -30,13 +31,13 @@ def chain(e, q, k, v, g, mask, H, T, d, alpha):
     return [x.numpy() for x in (o, dq, dk, dv)]
 
 
-def exact(q, k, v, g, mask, H, T, d, alpha):
+def exact(q, k, v, g, mask, H, T, d, alpha, alpha2=1.0):
     q, k, v, g = (x.astype(np.float64).reshape(H, d, T) for x in (q, k, v, g))
     s = alpha * np.matmul(q.transpose(0, 2, 1), k) + mask.astype(np.float64)
     p = np.exp(s - s.max(axis=2, keepdims=True))
     p /= p.sum(axis=2, keepdims=True)
     o = np.matmul(p, v.transpose(0, 2, 1))
-    dp = np.matmul(g.transpose(0, 2, 1), v)
+    dp = alpha2 * np.matmul(g.transpose(0, 2, 1), v)
     ds = p * (dp - (p * dp).sum(axis=2, keepdims=True)) * alpha
     dq = np.matmul(k, ds.transpose(0, 2, 1))
     return [o.reshape(H * T, d), dq.reshape(H * d, T), np.matmul(q, ds).reshape(H * d, T),
@@ -142,3 +143,37 @@ def test_tiny_gradients(hip, scale):
     quantum = 2.0 ** -149 * np.sqrt(got[3].size)
     for a, b in zip(got[1:], ref[1:]):
         assert np.linalg.norm(a.astype(np.float64) - b) <= TOL * np.linalg.norm(b) + T * quantum
+
+
+# lengths, head dims (32 and 64 wide tiles, one wave a SIMD at 128) and whether the forward keeps its score blocks
+WIDTHS = [(64, 64, True), (77, 64, True), (96, 32, True), (70, 128, True), (100, 64, False), (64, 32, False)]
+
+
+@pytest.fixture(scope="module")
+def no_blocks():
+    """An engine that keeps no score blocks: the key-line pass forms the scores."""
+    e = nnengine.Engine()
+    e.set_score_budget(0)
+    return e
+
+
+def chain_close(e, x, mask, H, T, d, alpha, alpha2=1.0):
+    ref = exact(*x, mask, H, T, d, alpha, alpha2)
+    assert all(np.abs(r).max() < 1e38 for r in ref)
+    for n, a, b in zip(("o", "dq", "dk", "dv"), chain(e, *x, mask, H, T, d, alpha, alpha2), ref):
+        assert np.isfinite(a).all(), n
+        # (T sums of values that may round to multiples of 2^-149)
+        assert np.linalg.norm(a - b) <= TOL * np.linalg.norm(b) + T * 2.0 ** -149 * np.sqrt(b.size), (n, rel(a, b))
+    return ref
+
+
+@pytest.mark.parametrize("T,d,keep", WIDTHS)
+def test_score_gradients_past_the_scaled_range(hip, no_blocks, T, d, keep):
+    """dO of 1e20 and V of 1e14: score gradients dS of 1e33 to 1e35, past 2^104, and finite products of them with Q
+    and K of about 1."""
+    rng = np.random.default_rng(T + d)
+    H = 2
+    q, k = normal(rng, (H * d, T)), normal(rng, (H * d, T))
+    v, g = normal(rng, (H * d, T)) * np.float32(1e14), normal(rng, (H * d, T)) * np.float32(1e20)
+    ref = chain_close(hip if keep else no_blocks, (q, k, v, g), causal_mask(T), H, T, d, d ** -0.5)
+    assert np.abs(ref[1]).max() > 2.0 ** 108
