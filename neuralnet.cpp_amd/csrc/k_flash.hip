@@ -616,6 +616,15 @@ __device__ __forceinline__ void value_parts(const typename VTile<DP>::Lds& tile,
     }
 }
 
+// The largest of |x| and big. (A NaN may be passed over.)
+__device__ __forceinline__ float max_abs(const f32x16& x, float big)
+{
+#pragma unroll
+    for (int r = 0; r < 16; r += 2)
+        big = __builtin_fmaxf(__builtin_fmaxf(__builtin_fabsf(x[r]), __builtin_fabsf(x[r + 1])), big);
+    return big;
+}
+
 // Not zero when one of x's values is not finite.
 __device__ __forceinline__ float not_finite(const f32x16& x, float sum)
 {
@@ -736,10 +745,11 @@ __device__ __forceinline__ float cell_scores(const f32x16& s, float alpha, const
 // (1536 cycles a cell and wave) beside about 250 vector instructions a cell
 // (scale, mask, max, exp2, and the weights' split), two waves a SIMD covering
 // each other: 48 KB of LDS and 2 workgroups a CU. A workgroup whose results
-// are not all finite, or whose scores are not in a row that has found no
-// weight yet (past the scaled range they are -inf as masked ones are), runs
-// its lines again with fwd_f32, the float32 chains, which take infinities and
-// NaN as they come.
+// or dot products are not all finite runs its lines again with fwd_f32, the
+// float32 chains, which take infinities and NaN as they come. (The dot
+// products have a check of their own, 8 instructions a cell: one that passes
+// the scaled range leaves a score of -inf, a masked key's, and finite
+// results.)
 template <int KP, int DP, bool WITH_O>
 struct FwdLds
 {
@@ -761,7 +771,7 @@ __device__ __forceinline__ bool fwd_split(const FlashFwdArgs& a, const FlashGeo&
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, h = lane >> 5, c = lane & 31;
     const int line = it.grp * kWaves + wave, qi = line * 32 + c;
     const SplitUnits su;
-    float mrun = kLowest, lrun = 0.0f, bad = 0.0f;
+    float mrun = kLowest, lrun = 0.0f, bad = 0.0f, big = 0.0f;
     f32x16 o[DU];
 #pragma unroll
     for (int u = 0; u < DU; ++u) o[u] = zero16();
@@ -836,7 +846,7 @@ __device__ __forceinline__ bool fwd_split(const FlashFwdArgs& a, const FlashGeo&
                     }
                     mrun = mnew;
                 }
-                if (__any(mrun == kLowest)) bad = not_finite(sc, bad);
+                big = max_abs(sc, big);
                 // Rows still without an allowed key keep lowest() and only -inf scores. (The split's scale
                 // is a product: an addend of 24 in the exponent costs it 4 bits.)
                 const float mb = mrun == kLowest ? 0.0f : mrun * kLog2e;
@@ -864,7 +874,7 @@ __device__ __forceinline__ bool fwd_split(const FlashFwdArgs& a, const FlashGeo&
         }
     }
     lrun += __shfl_xor(lrun, 32);
-    bad = __builtin_fmaf(lrun, 0.0f, bad);
+    bad = __builtin_fmaf(big, 0.0f, __builtin_fmaf(lrun, 0.0f, bad));
     if constexpr (WITH_O)
     {
 #pragma unroll

@@ -5,6 +5,7 @@
   float64. Bound: normwise 3e-6, about four times what float32 chains of this length show.
 * Inputs past the scaled range (2^104), keys excluded by -inf in K: the float32 chains.
 * Tiny gradients: no part is lost (the same bound). Score gradients past 2^104: float32 as well.
+* Dot products past 2^80 that alpha brings back to ordinary scores.
 """
 import numpy as np
 import pytest
@@ -177,3 +178,21 @@ def test_score_gradients_past_the_scaled_range(hip, no_blocks, T, d, keep):
     v, g = normal(rng, (H * d, T)) * np.float32(1e14), normal(rng, (H * d, T)) * np.float32(1e20)
     ref = chain_close(hip if keep else no_blocks, (q, k, v, g), causal_mask(T), H, T, d, d ** -0.5)
     assert np.abs(ref[1]).max() > 2.0 ** 108
+
+
+@pytest.mark.parametrize("T,d,keep", WIDTHS)
+@pytest.mark.parametrize("how", ["one_product", "cancelling", "negative_alpha"])
+def test_scores_whose_scaled_sums_overflow(hip, no_blocks, T, d, keep, how):
+    """Dot products below -2^80 (or with partial sums below it), infinite in the scaled sum, that alpha brings back
+    to scores of about 1: such a key weighs as much as any other. Every row finds an ordinary score first."""
+    rng = np.random.default_rng(T + d)
+    H, alpha = 2, 2.0 ** -81
+    q, k = np.zeros((H, d, T), np.float32), np.zeros((H, d, T), np.float32)
+    q[:, 0] = 2.0 ** 50
+    k[:, 0, 32:] = -(2.0 ** 31) * rng.uniform(0.75, 1.25, (H, T - 32))
+    if how == "cancelling":   # (in two steps of 16 dims)
+        q[:, 17], k[:, 17] = 2.0 ** 50, -0.375 * k[:, 0]
+    if how == "negative_alpha":
+        k, alpha = -k, -alpha
+    x = q.reshape(H * d, T), k.reshape(H * d, T), normal(rng, (H * d, T)), normal(rng, (H * d, T))
+    chain_close(hip if keep else no_blocks, x, causal_mask(T), H, T, d, alpha)
