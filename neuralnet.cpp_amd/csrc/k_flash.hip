@@ -625,6 +625,13 @@ __device__ __forceinline__ float max_abs(const f32x16& x, float big)
     return big;
 }
 
+// A scaled chain's factor alpha 2^-48 is a normal number, or zero: smaller ones would lose bits of alpha, so they
+// take the float32 chains.
+__device__ __forceinline__ bool factor_holds(float alpha)
+{
+    return alpha == 0.0f || __builtin_fabsf(alpha) >= 0x1p-78f;
+}
+
 // Not zero when one of x's values is not finite.
 __device__ __forceinline__ float not_finite(const f32x16& x, float sum)
 {
@@ -997,7 +1004,7 @@ __global__ __launch_bounds__(64 * kWaves, waves_per_simd(KP, DP)) void k_flash_f
     if ((threadIdx.x & 63) == 0) nz_s[threadIdx.x >> 6] = lw.nz;
     __syncthreads();
     const unsigned long long any = nz_s[0] | nz_s[1] | nz_s[2] | nz_s[3];
-    const bool bad = fwd_split<KP, DP, WITH_O, VDM, SST>(a, g, it, lw, any, L.s);
+    const bool bad = !factor_holds(a.alpha) || fwd_split<KP, DP, WITH_O, VDM, SST>(a, g, it, lw, any, L.s);
     if (__syncthreads_or(bad)) fwd_f32<KP, DP, WITH_O, VDM>(a, g, it, lw, any, L.f);
 }
 
@@ -1732,7 +1739,8 @@ __global__ __launch_bounds__(64 * kWaves, waves_per_simd(KP)) void k_flash_bwd_c
     const unsigned long long any = nz_s[0] | nz_s[1] | nz_s[2] | nz_s[3];
     if constexpr (SST || KP == 32)
     {
-        const bool bad = cols_split<KP, GDO, WDS, SST>(a, g, it.b, it.grp, it.rg, lw, any, L.s, St);
+        const bool bad = !((SST || factor_holds(a.alpha)) && factor_holds(a.alpha2)) ||
+                         cols_split<KP, GDO, WDS, SST>(a, g, it.b, it.grp, it.rg, lw, any, L.s, St);
         if (!__syncthreads_or(bad)) return;
     }
     cols_f32<KP, GDO, WDS, SST>(a, g, it.b, it.grp, it.rg, lw, any, L.f, St);

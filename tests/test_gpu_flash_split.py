@@ -6,6 +6,7 @@
 * Inputs past the scaled range (2^104), keys excluded by -inf in K: the float32 chains.
 * Tiny gradients: no part is lost (the same bound). Score gradients past 2^104: float32 as well.
 * Dot products past 2^80 that alpha brings back to ordinary scores.
+* Factors alpha whose product with the scale is no normal number.
 """
 import numpy as np
 import pytest
@@ -196,3 +197,13 @@ def test_scores_whose_scaled_sums_overflow(hip, no_blocks, T, d, keep, how):
         k, alpha = -k, -alpha
     x = q.reshape(H * d, T), k.reshape(H * d, T), normal(rng, (H * d, T)), normal(rng, (H * d, T))
     chain_close(hip if keep else no_blocks, x, causal_mask(T), H, T, d, alpha)
+
+
+@pytest.mark.parametrize("T,d,keep", WIDTHS)
+def test_small_factors(hip, no_blocks, T, d, keep):
+    """alpha and the dP product's alpha below 2^-78: times the split's 2^-48 they are no normal numbers."""
+    rng = np.random.default_rng(T + d)
+    H, alpha, alpha2 = 2, float(np.float32(1.2345e-24)), float(np.float32(1.2345e-29))
+    q, k = normal(rng, (H * d, T)) * np.float32(1e11), normal(rng, (H * d, T)) * np.float32(1e11)
+    v, g = normal(rng, (H * d, T)), normal(rng, (H * d, T)) * np.float32(1e20)
+    chain_close(hip if keep else no_blocks, (q, k, v, g), causal_mask(T), H, T, d, alpha, alpha2)
