@@ -8,6 +8,7 @@
 * Inputs whose parts overflow when scaled, infinities, NaN, results past 2^80: the float32 path
   that those outputs are formed again on (same classification as float64 rounded to float32).
 * Tiny and denormal inputs: no part is lost (the same bound).
+* K of 1 and 2: the float32 cores' roundings.
 * Sums over operands by sequence and in segments whose lengths are 16 mod 32 (half a stage).
 """
 import ctypes
@@ -95,6 +96,21 @@ def test_tiny_values(hip, sa, sb):
     A = (uniform(rng, (M, K)).astype(np.float64) * sa).astype(np.float32)
     B = (uniform(rng, (K, N)).astype(np.float64) * sb).astype(np.float32)
     check(hip.matmul(hip.tensor(A), hip.tensor(B)).numpy(), A, B)
+
+
+@pytest.mark.parametrize("M,N", [(3, 5), (64, 129), (300, 500), (1100, 2100)])
+@pytest.mark.parametrize("tA,tB", [(False, False), (True, False), (False, True), (True, True)])
+def test_one_and_two_products(hip, M, N, tA, tB):
+    """K = 1: each product rounded once. K = 2: at most two roundings, of a product and of the sum."""
+    rng = np.random.default_rng(M)
+    for K in (1, 2):
+        A, B = (rng.normal(0, 1, s).astype(np.float32) for s in ((M, K), (K, N)))
+        C = hip.matmul(hip.tensor(A.T if tA else A), hip.tensor(B.T if tB else B), tA, tB).numpy()
+        if K == 1:
+            assert np.array_equal(C, A * B)
+        else:
+            A, B = A.astype(np.float64), B.astype(np.float64)
+            assert np.all(np.abs(C - A @ B) <= 2 * 2.0 ** -24 * (np.abs(A) @ np.abs(B)))
 
 
 class BySeq(ctypes.Structure):
