@@ -33,6 +33,7 @@
 //   D: 16 values, value r at row 8*(r/4) + 4*(l/32) + r%4, column l%32.
 #include <cmath>
 #include <mutex>
+#include <type_traits>
 
 #include "common.hpp"
 #include "nnhip_kernels.h"
@@ -436,31 +437,56 @@ __global__ __launch_bounds__(64 * WM * WN, FM * FN == 4 ? 2 : 3) void k_gemm(
             }
     if (K <= 2 || __any(check != 0.0f))
     {
-        const int am = m0 + al, bn = n0 + bl;
+        // Loads straight to registers, without LDS and its barriers, which the other waves are past. 16 k a step:
+        // a lane's 8 are one run of its line where k is contiguous, else each a run of the wave's lines, and MFMA
+        // e sums k + e of both lane halves. What it costs, for 6144 x 8192 x 768 and 768 x 8192 x 6144 (TN), us:
+        // all outputs NaN 1161 and 1220 (float32 kernels 599 and 634, two k a step 3200 and 3568), one NaN in A
+        // 652 and 610 (667 and 704; 1803 and 1161), none 489 and 524 (691 and 707).
+        auto eight = [&](auto kc, const float* q, long ld, int left, float* x) {
+            const long step = decltype(kc)::value ? 1 : ld;
+            if (left >= 8)
+            {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) x[e] = q[e * step];
+            }
+            else
+            {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) x[e] = e < left ? q[e * step] : 0.0f;
+            }
+        };
 #pragma unroll
         for (int i = 0; i < FM; ++i)
 #pragma unroll
+            for (int j = 0; j < FN; ++j) acc[i][j] = floatx16{};
+        for (int k0 = k_lo; k0 < k_hi; k0 += 16)
+        {
+            const int k = k0 + 8 * kl;
+            const float* ap = seg_a(A, k);
+            const float* bp = seg_b(B, k) + b_off;
+            const long ka = seg_a.within(k) + (SEG && !TA && sa_t ? (long)(k / sa_t) * sa_d : 0);
+            const long kb = seg_b.within(k) + (SEG && TB && sb_t ? (long)(k / sb_t) * sb_d : 0);
+            float a[FM][8], b[FN][8];
+#pragma unroll
+            for (int i = 0; i < FM; ++i)
+            {
+                const long gm = min(m0 + al + 32 * i, M - 1);
+                eight(std::bool_constant<!TA>{}, TA ? ap + ka * lda + gm : ap + gm * lda + ka, lda, k_hi - k, a[i]);
+            }
+#pragma unroll
             for (int j = 0; j < FN; ++j)
             {
-                floatx16 c = {};
-                const long gm = min(am + 32 * i, M - 1), gn = min(bn + 32 * j, N - 1);
-                for (int k0 = k_lo; k0 < k_hi; k0 += 2)
-                {
-                    const int k = k0 + kl;
-                    float a = 0.0f, b = 0.0f;
-                    if (k < k_hi)
-                    {
-                        const float* ap = seg_a(A, k);
-                        const float* bp = seg_b(B, k) + b_off;
-                        const long ka = seg_a.within(k) + (SEG && !TA && sa_t ? (long)(k / sa_t) * sa_d : 0);
-                        const long kb = seg_b.within(k) + (SEG && TB && sb_t ? (long)(k / sb_t) * sb_d : 0);
-                        a = TA ? ap[ka * lda + gm] : ap[gm * lda + ka];
-                        b = TB ? bp[gn * ldb + kb] : bp[kb * ldb + gn];
-                    }
-                    c = __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
-                }
-                acc[i][j] = c;
+                const long gn = min(n0 + bl + 32 * j, N - 1);
+                eight(std::bool_constant<TB>{}, TB ? bp + gn * ldb + kb : bp + kb * ldb + gn, ldb, k_hi - k, b[j]);
             }
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+#pragma unroll
+                for (int i = 0; i < FM; ++i)
+#pragma unroll
+                    for (int j = 0; j < FN; ++j)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i][e], b[j][e], acc[i][j], 0, 0, 0);
+        }
     }
 
     // Epilogue: C = alpha * acc, then + bias[row] and / or + C (each rounded

@@ -9,7 +9,8 @@
   that those outputs are formed again on (same classification as float64 rounded to float32).
 * Tiny and denormal inputs: no part is lost (the same bound).
 * K of 1 and 2: the float32 cores' roundings.
-* Sums over operands by sequence and in segments whose lengths are 16 mod 32 (half a stage).
+* Sums over operands by sequence and in segments whose lengths are 16 mod 32 (half a stage), with
+  K split inside a sequence or segment, and with infinities in them.
 """
 import ctypes
 
@@ -153,3 +154,98 @@ def test_by_sequence_of_half_stages(hip, T, nseq):
     check(c.numpy(), G, X.T)
     ref = G.astype(np.float64).sum(1, keepdims=True)
     assert np.all(np.abs(rows.numpy() - ref) <= K * 2.0 ** -24 * np.abs(G).astype(np.float64).sum(1, keepdims=True))
+
+
+def check_class(C, A, B):
+    """check, and where the float64 result is not finite its class."""
+    A, B = A.astype(np.float64), B.astype(np.float64)
+    with np.errstate(invalid="ignore"):
+        ref = A @ B
+    same_class(C, ref)
+    fin = np.isfinite(ref)
+    b = bound(np.where(np.isfinite(A), A, 0.0), np.where(np.isfinite(B), B, 0.0), A.shape[1])
+    assert np.all(np.abs(C[fin] - ref[fin]) <= b[fin] + 2.0 ** -149)
+
+
+@pytest.fixture
+def lib(hip):
+    l, P, SZ, F, I = hip._lib, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_float, ctypes.c_int
+    l.nnhip_gemm_workspace_bytes.restype, l.nnhip_gemm_workspace_bytes.argtypes = SZ, [SZ] * 4
+    l.nnhip_engine_stream.restype, l.nnhip_engine_stream.argtypes = P, [P]
+    l.nnhip_gemm_tn_sum.argtypes = [P, P, SZ, P, SZ, SZ, SZ, F, P, SZ, P]
+    l.nnhip_gemm_tn_sum_seq.argtypes = [P, P, SZ, P, SZ, SZ, SZ, F, BySeq, P, SZ, P]
+    l.nnhip_gemm_epilogue_seq.argtypes = [P, P, P, SZ, SZ, SZ, F, P, I, BySeq, P, SZ, P]
+    l.nnhip_gemm_group_acc_seq.argtypes = [P, P, P, SZ, SZ, SZ, SZ, I, I, P, I, P, P, P, SZ, P]
+    return l
+
+
+def by_seq(hip, X, T):
+    """X (d, K) as heads' rows: per sequence of T columns its (d, T)."""
+    d = X.shape[0]
+    return hip.tensor(np.ascontiguousarray(X.reshape(d, -1, T).transpose(1, 0, 2)).reshape(-1, T))
+
+
+@pytest.mark.parametrize("klen,split", [(48, False), (1040, True), (688, True)])
+@pytest.mark.parametrize("bad", [False, True])
+def test_segments(hip, lib, klen, split, bad):
+    """Three segments, with K split across them, and with an infinity in one (the float32 path)."""
+    M, N = 132, 260
+    rng = np.random.default_rng(klen)
+    A, B = [uniform(rng, (klen, M)) for _ in range(3)], [uniform(rng, (klen, N)) for _ in range(3)]
+    if bad:
+        A[1][klen - 1, 70], B[2][17, 200] = np.inf, np.nan
+    a, b, c = [hip.tensor(x) for x in A], [hip.tensor(x) for x in B], hip.create_tensor(M, N)
+    wsb = lib.nnhip_gemm_workspace_bytes(M, N, 3 * klen, 1) if split else 0
+    assert (wsb > 0) == split
+    ws = hip.create_tensor(1, max(wsb // 4, 1))
+    assert lib.nnhip_gemm_tn_sum(_ptrs(a), _ptrs(b), 3, c.data_ptr(), M, N, klen, 1.0, ws.data_ptr() if wsb else None,
+                                 wsb, lib.nnhip_engine_stream(hip._e)) == 0
+    check_class(c.numpy(), np.concatenate(A).T, np.concatenate(B))
+
+
+@pytest.mark.parametrize("T,nseq,split", [(48, 6, False), (16, 130, True), (48, 50, True), (80, 27, True)])
+@pytest.mark.parametrize("bad", [False, True])
+def test_by_sequence(hip, lib, T, nseq, split, bad):
+    """Two weight gradients G X^T of rows by sequence with their row sums: K split inside a sequence (k slices are
+    multiples of 32, sequences of 16), and an infinity."""
+    d, K, n = 128, T * nseq, 2
+    rng = np.random.default_rng(T)
+    G, X = [uniform(rng, (d, K)) for _ in range(n)], [uniform(rng, (d, K)) for _ in range(n)]
+    if bad:
+        G[0][70, K - 3], X[1][5, T + 1] = np.inf, -np.inf
+    g, x = [by_seq(hip, a, T) for a in G], [by_seq(hip, a, T) for a in X]
+    c, rows = [hip.tensor(np.zeros((d, d))) for _ in range(n)], [hip.tensor(np.zeros((d, 1))) for _ in range(n)]
+    lay = (BySeq * n)(*[BySeq(T, d * T)] * n)
+    wsb = lib.nnhip_gemm_workspace_bytes(d, d, K, n) if split else 0
+    assert (wsb > 0) == split
+    ws = hip.create_tensor(1, max(wsb // 4, 1))
+    assert lib.nnhip_gemm_group_acc_seq(_ptrs(g), _ptrs(x), _ptrs(c), n, d, d, K, 1, 1, _ptrs(rows), 1, lay, lay,
+                                        ws.data_ptr() if wsb else None, wsb, lib.nnhip_engine_stream(hip._e)) == 0
+    for i in range(n):
+        check_class(c[i].numpy(), G[i], X[i].T)
+        ref, r = G[i].astype(np.float64).sum(1, keepdims=True), rows[i].numpy()
+        same_class(r, ref)
+        fin = np.isfinite(ref)
+        assert np.all(np.abs(r[fin] - ref[fin]) <= (K * 2.0 ** -24 * np.abs(G[i]).astype(np.float64).sum(1, keepdims=True))[fin])
+
+
+@pytest.mark.parametrize("bad", [False, True])
+@pytest.mark.parametrize("n", [1, 2])
+def test_columns_by_sequence(hip, lib, n, bad):
+    """B by sequence, untransposed: W X and a sum of two W^T X."""
+    M, K, T, nseq = 128, 48, 128, 3
+    rng = np.random.default_rng(n)
+    A, B = [uniform(rng, (K, M)) for _ in range(n)], [uniform(rng, (K, T * nseq)) for _ in range(n)]
+    if bad:
+        A[0][40, 9], B[n - 1][3, T + 70] = np.nan, np.inf
+    b, c, st = [by_seq(hip, x, T) for x in B], hip.create_tensor(M, T * nseq), lib.nnhip_engine_stream(hip._e)
+    if n == 1:
+        a = hip.tensor(A[0].T)
+        rc = lib.nnhip_gemm_epilogue_seq(a.data_ptr(), b[0].data_ptr(), c.data_ptr(), M, T * nseq, K, 1.0, None, 0,
+                                         BySeq(T, K * T), None, 0, st)
+    else:
+        a = [hip.tensor(x) for x in A]
+        rc = lib.nnhip_gemm_tn_sum_seq(_ptrs(a), _ptrs(b), n, c.data_ptr(), M, T * nseq, K, 1.0, BySeq(T, K * T), None,
+                                       0, st)
+    assert rc == 0
+    check_class(c.numpy(), np.concatenate(A).T, np.concatenate(B))
