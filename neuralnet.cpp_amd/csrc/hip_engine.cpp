@@ -1886,7 +1886,6 @@ Result<Tensor> HipEngine::from_matrix(const Matrix& m)
 Result<Matrix> HipEngine::to_matrix(const Tensor& t)
 {
     if (!t.is_gpu()) return fail("to_matrix: tensor is not GPU");
-    NN_CHECK(settle_reads_({&t}));
     Matrix m(t.rows(), t.cols());
     NN_CHECK(read_into(t, m.data()));
     return m;
@@ -1900,10 +1899,10 @@ Result<Matrix> HipEngine::to_matrix(const Tensor& t)
 Result<void> HipEngine::read_into(const Tensor& t, Scalar* out)
 {
     if (!t.is_gpu()) return fail("to_matrix: tensor is not GPU");
+    std::lock_guard<std::mutex> lk(read_mu_);
     NN_CHECK(settle_reads_({&t}));
     const std::size_t bytes = t.size() * sizeof(float);
     auto s = static_cast<hipStream_t>(stream_);
-    std::lock_guard<std::mutex> lk(read_mu_);
     if (bytes && !read_stage_)
     {
         for (void*& e : read_ev_)

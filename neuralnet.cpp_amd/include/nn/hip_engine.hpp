@@ -382,7 +382,9 @@ private:
     // Two pinned slots for reads (read_into): while one is copied out to the
     // caller's memory the other is being filled.
     static constexpr std::size_t kReadSlot = std::size_t(2) << 20;
-    std::mutex read_mu_;   // the slots serve one read at a time, also from several threads
+    // One read at a time, from several threads too: they share the slots and the records that a read launches. (An
+    // engine's other calls stay its caller's to order.)
+    std::mutex read_mu_;
     void* read_stage_ = nullptr;
     void* read_ev_[2] = {nullptr, nullptr};
 

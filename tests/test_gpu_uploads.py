@@ -4,9 +4,12 @@ from_matrix and copy_from (compute_engine.hpp) copy small host data into a slot
 of a pinned staging ring and return once the upload is queued (no wait for the
 stream); larger data is uploaded and waited for. Checked: more uploads than the
 ring has slots, each read back after all of them, against the host data bit for
-bit; copy_from into a tensor that queued work still reads; the large path; and
-transposes of row and column vectors (plain copies of the same floats).
+bit; copy_from into a tensor that queued work still reads; the large path;
+transposes of row and column vectors (plain copies of the same floats); and
+reads around the sizes of the pinned read slots and from several threads.
 """
+from concurrent.futures import ThreadPoolExecutor
+
 import numpy as np
 import pytest
 
@@ -49,3 +52,24 @@ def test_vector_transpose(hip, shape):
     rng = np.random.default_rng(4)
     X = normal(rng, shape)
     assert np.array_equal(hip.transpose(hip.tensor(X)).numpy().view(np.uint32), X.T.copy().view(np.uint32))
+
+
+@pytest.mark.parametrize("n", [1, (1 << 19) - 1, 1 << 19, (1 << 19) + 1, (1 << 20) - 1, 1 << 20, 5 * (1 << 19) + 3])
+def test_reads_around_the_slots(hip, n):
+    """Reads of up to one pinned slot (2 MiB), of whole slots and of slots and a rest."""
+    x = normal(np.random.default_rng(n), (1, n))
+    assert np.array_equal(hip.tensor(x).numpy().view(np.uint32), x.view(np.uint32))
+
+
+def test_reads_from_several_threads(hip):
+    """Results that are still recorded, small ones and ones of several slots, read by four threads at once: each read
+    launches what it needs and passes through the slots by itself."""
+    rng = np.random.default_rng(4)
+    X = [normal(rng, s) for s in ((700, 1100), (64, 32), (1500, 900), (33, 65))]
+    W = [normal(rng, (a.shape[0], a.shape[0])) for a in X]
+    ref = [w.astype(np.float64) @ x.astype(np.float64) for w, x in zip(W, X)]
+    with ThreadPoolExecutor(4) as pool:
+        for _ in range(10):
+            out = [hip.matmul(hip.tensor(w), hip.tensor(x)) for w, x in zip(W, X)]
+            for got, r in zip(pool.map(lambda t: t.numpy(), out), ref):
+                assert np.abs(got - r).max() <= 1e-4 * np.abs(r).max()
