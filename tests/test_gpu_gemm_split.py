@@ -7,7 +7,7 @@
   |dC| <= (6 ceil(K / 16) + 8) 2^-24 (|A||B|)_ij.
 * Inputs whose parts overflow when scaled, infinities, NaN, results past 2^80: the float32 path
   that those outputs are formed again on (same classification as float64 rounded to float32).
-* Tiny and denormal inputs: no part is lost (the same bound).
+* Tiny and denormal inputs, inputs of 2^87 to 2^103: no part is lost (the same bound).
 * K of 1 and 2: the float32 cores' roundings.
 * Sums over operands by sequence and in segments whose lengths are 16 mod 32 (half a stage), with
   K split inside a sequence or segment, and with infinities in them.
@@ -97,6 +97,20 @@ def test_tiny_values(hip, sa, sb):
     A = (uniform(rng, (M, K)).astype(np.float64) * sa).astype(np.float32)
     B = (uniform(rng, (K, N)).astype(np.float64) * sb).astype(np.float32)
     check(hip.matmul(hip.tensor(A), hip.tensor(B)).numpy(), A, B)
+
+
+@pytest.mark.parametrize("M,N,K", [(5, 6, 3), (130, 140, 77), (300, 1500, 33), (100, 90, 2600)])
+@pytest.mark.parametrize("large", ["A", "B"])
+def test_large_values_within_the_scaled_range(hip, M, N, K, large):
+    """One operand spread over 2^87 to 2^103, just below the inputs whose parts overflow when scaled, the other so
+    small that results stay below 2^80: the bf16 parts, exact there too."""
+    rng = np.random.default_rng(K)
+    B = uniform(rng, (K, N)) * np.float32(2.0 ** -40)
+    A = (2.0 ** rng.uniform(87, 103, (M, K)) * rng.choice([-1.0, 1.0], (M, K))).astype(np.float32)
+    if large == "B":
+        A, B = np.ascontiguousarray(B.T), np.ascontiguousarray(A.T)
+    check(hip.matmul(hip.tensor(A), hip.tensor(B)).numpy(), A, B)
+    check(hip.matmul(hip.tensor(A), hip.tensor(B.T), False, True).numpy(), A, B)
 
 
 @pytest.mark.parametrize("M,N", [(3, 5), (64, 129), (300, 500), (1100, 2100)])
