@@ -92,8 +92,8 @@ inline size_t score_blocks_floats(size_t batch, size_t M, size_t N)
     return batch * ((M + 31) / 32) * ((N + 31) / 32) * 1024;
 }
 
-// Shapes the one-pass kernels take: head dims K (and Kd) <= 64, value width
-// D <= 64 with D % 4 == 0. The backward also needs K % 4 == 0 and ldg % 4 == 0.
+// Shapes the one-pass kernels take: head dims K (and Kd) <= 128, value width
+// D <= 128 with D % 4 == 0. The backward also needs K % 4 == 0 and ldg % 4 == 0.
 bool flash_supported(size_t batch, size_t M, size_t N, size_t K, size_t D);
 // Mask cell table: one byte per 32x32 cell of each (M, N) mask (0 all -inf, 1 all zero, 2 general);
 // masks batches, mask_bs floats apart, give batches tables of flash_cells_bytes(M, N) each.

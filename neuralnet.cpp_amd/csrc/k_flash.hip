@@ -416,9 +416,13 @@ __device__ __forceinline__ void line_operand(const float* base, int dims, int T,
 //     score registers 8 s .. 8 s + 7 of step s, tokens 16 s + 4 h + 0..3 and
 //     + 8..11: the octet 2 s + h holds those tokens, so weights never move
 //     between lanes. Row u 32 + i holds dim DU i + u (the outputs' order).
-// Rows of 64 or 128 bytes, octets swapped so that neither the 16-byte reads of
-// neighbouring rows' same octet (16 lanes at a time) nor the writes (8 lanes)
-// meet an LDS bank twice. A cell of KP = DP = 64 is 48 MFMAs of 32
+// Rows of 64 or 128 bytes, octets swapped so that the 16-byte reads of
+// neighbouring rows' same octet (16 lanes at a time) and the score form's
+// writes (8 lanes) meet no LDS bank twice. The value form's writes do for 64
+// and 128 dims: neighbouring dims lie 32 rows, 2048 bytes, apart, so two lanes
+// share a bank (four where 128 dims are staged from rows of tokens). By the
+// counters conflicts are 15, 16 and 26 % of the LDS cycles of the forward, the
+// key-line pass and the dQ pass of a 12-layer training step. A cell of KP = DP = 64 is 48 MFMAs of 32
 // cycles forward where the float32 chains take 64 of 64.
 typedef bf16x8 Parts[3];
 

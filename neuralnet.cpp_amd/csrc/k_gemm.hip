@@ -764,8 +764,10 @@ __global__ __launch_bounds__(256) void k_splitk_reduce(const float* __restrict__
 
 // What callers are told about a product before it runs: whole tiles for
 // operands by sequence (bm, bn), and the split-K partials that a workspace is
-// sized for and that nnhip_gemm_noalloc's scratch is compared with. Fixed by
-// the shape alone; the launch's own tiles and splits (plan_gemm) stay within.
+// sized for and that nnhip_gemm_noalloc's scratch is compared with. These are
+// the entry points' rules, by the shape alone and older than the tiles in use:
+// what they take, refuse and ask for must not move with the planner. The
+// launch's own tiles and splits (plan_gemm) stay within.
 struct Terms
 {
     int bm, bn, splits;
@@ -853,8 +855,13 @@ constexpr Tile kTiles[3] = {{256, 128, 1, {2.35, 0, 0}, 6.0},
 
 // The tile and split with the least estimated time: the stages of the CU with
 // the most workgroups, the stores, and for split K the partials' sum (3 us and
-// its bytes at 5.5 TB/s). The estimate picks within 2 % of the best measured
-// one on average over those 62. Partials take at most `budget` bytes; K below
+// its bytes at 5.5 TB/s). Over another 62 products, of 128..32000 in each
+// dimension, it picks within 1.4 % of the best measured one on average, 21 % at
+// worst; one tile for all of them, each with its best split, loses 15 to 30 %. The
+// constants beside the stage times are fitted, and matter less than they look:
+// without the overlap factor the average is 0.7 %, without the store term
+// 1.4 %, without the fixed parts 1.6 %, without the partials' bytes 3.8 %.
+// Partials take at most `budget` bytes; K below
 // 1024 is never split (a product and its heads-layout form sum alike there).
 constexpr size_t kSplitBudget = NNHIP_GEMM_NOALLOC_SCRATCH_BYTES;
 Plan plan_gemm(size_t M, size_t N, size_t K, size_t batch, size_t budget)
@@ -1396,7 +1403,9 @@ int gemm_dispatch(const float* A, const float* B, float* C, size_t M, size_t N, 
     {
         Terms w = gemm_terms(M, N, K, batch, workspace != nullptr);
         if (need(w.splits) > ws_bytes) w = gemm_terms(M, N, K, batch, false);
-        // whole tiles, 16-byte loads, and no tile or stage across two sequences
+        // What callers may count on being refused or taken, from the shape and the alignment alone (gemm_terms). The
+        // kernel itself needs less: 4-byte alignment, 8 k of a line in one sequence, and, for an untransposed B by
+        // sequence, a tile's columns in one.
         const GemmGroup& g = e.grp ? *e.grp : e.seg ? *e.seg : *e.sq;
         const bool whole = M % w.bm == 0 && N % w.bn == 0 && K % 16 == 0 && lda % 4 == 0 && ldb % 4 == 0 &&
                            sA % 4 == 0 && sB % 4 == 0 && aligned16(A) && aligned16(B);
@@ -1559,7 +1568,7 @@ int group_acc(const float* const* A, const float* B, const float* const* B_each,
             g.bS[i] = static_cast<long>(b_seq[i].step);
             by_seq = true;
         }
-        // members' loads are 16-byte loads when member 0's are
+        // (a rule of the entry point: the loads need 4-byte alignment only)
         if (!aligned16(A[i]) || (B_each && !aligned16(B_each[i]))) return -1;
     }
     rs.acc = row_sums_accumulate ? 1 : 0;
